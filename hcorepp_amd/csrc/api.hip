@@ -450,7 +450,7 @@ hcorepp_status recompress_plain(hcorepp_ctx *ctx, T alpha, const Holder<T> &ad, 
     }
     int32_t *jflags = (int32_t *) arena_take(ctx, sizeof(int32_t) * JACOBI_MAX_SWEEPS);
     T *vpan = (T *) arena_take(ctx, sizeof(T) * ((size_t) std::max(m, n) * 16 + 1024));
-    HIP_TRY(launch_recomp_pre<T>(s, d, K, kLdsBytes, pb, jflags, reinterpret_cast<int32_t *>(ctx->pinned + HDR_WORDS),
+    HIP_TRY(launch_recomp_pre<T>(s, d, K, kLdsBytes, pb, jflags, ctx->pinned + HDR_WORDS,
                                  vpan));
     // The plain form reads the new rank back with one stream synchronisation,
     // as the reference does (src/kernels/cuda/CudaKernels.cu:656-697).

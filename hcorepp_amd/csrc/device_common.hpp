@@ -257,8 +257,57 @@ __device__ __forceinline__ int wave_multi_sum_index(int l) {
     return l >> (6 - log2_const<NV>());
 }
 
+// Lane that holds value index j after wave_multi_sum<NV>: index bits map to lane bits 5..(6-log2 NV).
+template <int NV>
+__device__ __forceinline__ constexpr int multi_sum_src_lane(int j) {
+    return j << (6 - log2_const<NV>());
+}
+
 // Accumulator of one FP64 matrix-core operation (v_mfma_f64_16x16x4f64): four doubles per lane.
 typedef double hcamd_doublex4 __attribute__((ext_vector_type(4)));
+
+typedef float hcamd_floatx4 __attribute__((ext_vector_type(4)));
+
+// One 16 x 16 x 4 matrix-core operation: A[i][k] in lane i + 16 k, B[k][j] in lane j + 16 k; element v
+// of lane l of the accumulator is D[row(v, l / 16)][l % 16] (FP64: row groups of one, FP32: of four).
+template <typename T>
+struct Mfma16;
+template <>
+struct Mfma16<double> {
+    using acc = hcamd_doublex4;
+    static __device__ __forceinline__ acc zero() { return acc{0.0, 0.0, 0.0, 0.0}; }
+    static __device__ __forceinline__ acc mma(double a, double b, acc c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ constexpr int row(int v, int k4) { return 4 * v + k4; }
+};
+template <>
+struct Mfma16<float> {
+    using acc = hcamd_floatx4;
+    static __device__ __forceinline__ acc zero() { return acc{0.f, 0.f, 0.f, 0.f}; }
+    static __device__ __forceinline__ acc mma(float a, float b, acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ constexpr int row(int v, int k4) { return 4 * k4 + v; }
+};
+
+// Value of lane `src` (any lane, per-lane choice) in this lane, through the LDS crossbar.
+__device__ __forceinline__ float lane_fetch(float v, int src) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(4 * src, __float_as_int(v)));
+}
+__device__ __forceinline__ double lane_fetch(double v, int src) {
+    const int lo = __builtin_amdgcn_ds_bpermute(4 * src, __double2loint(v));
+    const int hi = __builtin_amdgcn_ds_bpermute(4 * src, __double2hiint(v));
+    return __hiloint2double(hi, lo);
+}
+
+// Order this wave's LDS accesses before and after it (a wave's LDS operations complete in order, so
+// only the compiler has to be kept from moving them): for data that lanes of one wave exchange
+// through LDS of their own, without a workgroup barrier.
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 // dst[e] = src[e] for e in [0, n) by the whole workgroup, four loads in flight per thread.
 template <typename T>

@@ -217,7 +217,6 @@ __device__ void wg_gemm(int M, int N, int Kd, T alpha, const T *A, int64_t lda, 
 // MFMA lane layout (16x16x4): A[i][k] from lane i + 16 k, B[k][j] from lane j + 16 k,
 // D[4 (l / 16) + v][l % 16] in element v of lane l.
 // ---------------------------------------------------------------------------
-typedef float hcamd_floatx4 __attribute__((ext_vector_type(4)));
 constexpr int MS_BITS = 10, MS_SLICES = 4;
 constexpr int GTM_SLICE_A = GT_K * (GT_M + 1), GTM_SLICE_B = GT_K * (GT_N + 1);
 constexpr int GTM_LDS_FLOATS = MS_SLICES * (GTM_SLICE_A + GTM_SLICE_B) + GT_M + GT_N;

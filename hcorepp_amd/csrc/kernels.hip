@@ -4,6 +4,8 @@
 // one update in one workgroup and pulls updates from a device work queue.
 #include "kernels.hpp"
 
+#include <cstring>
+
 namespace hcamd {
 
 
@@ -41,13 +43,6 @@ template <typename T>
 __global__ void HCAMD_KERNEL k_y(RecompDesc<T> d) {
     __shared__ T lds[GT_LDS_ELEMS];
     ph_y<T>(d, blockIdx.x, gridDim.x, lds);
-}
-
-template <typename T>
-__global__ void HCAMD_KERNEL k_svd(RecompDesc<T> d) {
-    __shared__ T gbuf[JACOBI_LDS_ELEMS];
-    ph_core<T>(d, gbuf);
-    ph_svd<T>(d, gbuf);
 }
 
 // ---------------------------------------------------------------------------
@@ -204,18 +199,18 @@ static hipError_t launch_qr_mw(hipStream_t s, const RecompDesc<T> &d, int64_t ld
 }
 
 // ---------------------------------------------------------------------------
-// Multi-workgroup core SVD of the plain (one update per launch sequence) form.  A large core
-// (hundreds of columns) is the whole cost of an update, so its one-sided block Jacobi is spread
-// over the GPU: each launch is one step of the round-robin ordering of column blocks, one
-// workgroup per block pair (the four waves of a workgroup share the pair's 16 columns, rows
-// split across the waves).  flags[s] records whether sweep s rotated anything; the launches of
-// a later sweep return at once when the previous sweep was already rotation-free.
+// Core SVD of the plain (one update per launch sequence) form: the core build, the Jacobi with V
+// accumulated, the rank rule.  Narrow cores run the Jacobi in one workgroup; a core of MW_MIN_COLS
+// columns or more is spread over the GPU, one launch per step of the round-robin ordering of
+// super-blocks (jacobi.hpp).  flags[s] records whether sweep s saw a pair far from orthogonal; the
+// launches of a later sweep return at once when it did not.
 // ---------------------------------------------------------------------------
-constexpr int MW_TW = 16;
+constexpr int JW_THREADS = 512;                  // the one-workgroup Jacobi
+constexpr int64_t JW_LDS_BYTES = 150 * 1024;     // its LDS: the workgroup has the CU to itself
 
 template <typename T>
 __global__ void HCAMD_KERNEL k_core(RecompDesc<T> d, int32_t *flags) {
-    __shared__ T gbuf[JACOBI_LDS_ELEMS];
+    __shared__ T gbuf[CORE_LDS_ELEMS];
     ph_core<T>(d, gbuf);
     for (int i = threadIdx.x; i < JACOBI_MAX_SWEEPS; i += NT) flags[i] = 0;
     if (threadIdx.x == 0) {
@@ -227,44 +222,109 @@ __global__ void HCAMD_KERNEL k_core(RecompDesc<T> d, int32_t *flags) {
     }
 }
 
-template <typename T, int RPL>
-__global__ void HCAMD_KERNEL k_jacobi_step(RecompDesc<T> d, int32_t *flags, int sweep, int step) {
-    constexpr int B = MW_TW / 2;
-    __shared__ T lds[coop_rec_lds_elems<T, MW_TW>()];
-    if (sweep > 0 && flags[sweep - 1] == 0) return;  // converged in an earlier sweep
+// One-workgroup Jacobi; J, and V beside it, move into LDS where they fit (ld odd).
+template <typename T>
+__global__ void __launch_bounds__(JW_THREADS) k_jacobi_wg(RecompDesc<T> d) {
+    extern __shared__ unsigned char smem_raw[];
+    T *lds = reinterpret_cast<T *>(smem_raw);
+    constexpr int NW = JW_THREADS / WAVE;
+    constexpr int64_t cap = JW_LDS_BYTES / (int64_t) sizeof(T) - gram_jacobi_lds<T>(NW);
     Ws<T> w = ws_of(d);
     const Dims z = dims_of(d, w);
-    const int rows = z.mu, ncols = z.kt;
-    if (ncols <= 1) return;
-    const int nblk = (ncols + B - 1) / B;
-    const int nbp = nblk + (nblk & 1);
-    const int bp = (int) blockIdx.x;
-    if (step >= nbp - 1 || bp >= nbp / 2) return;
-    int bI, bJ;
-    if (bp == 0) {
-        bI = nbp - 1;
-        bJ = step;
+    const int rows = z.mu, nc = z.kt, ldj = rows | 1, ldv = nc | 1;
+    if (rows > JACOBI_ROWS_MAX) {
+        if (threadIdx.x == 0) w.hdr[HDR_STATUS] |= STATUS_TOO_BIG;
+        return;
+    }
+    const T fro2 = (T) __longlong_as_double(w.hdr[HDR_JFRO2]), stop = JacobiStopCos<T>::tight;
+    T *Jl = lds + gram_jacobi_lds<T>(NW), *Vl = Jl + (int64_t) ldj * nc;
+    const bool jin = (int64_t) ldj * nc <= cap, vin = (int64_t) (ldj + ldv) * nc <= cap;
+    int sweeps;
+    if (nc < 1) {
+        sweeps = 0;
+    } else if (jin) {
+        for (ColWalk p(threadIdx.x, JW_THREADS, rows); p.c < nc; p.next())
+            Jl[p.i + p.c * ldj] = w.j[p.i + (int64_t) p.c * rows];
+        if (vin) {
+            for (ColWalk p(threadIdx.x, JW_THREADS, nc); p.c < nc; p.next()) Vl[p.i + p.c * ldv] = T(p.i == p.c);
+            __syncthreads();
+            sweeps = wg_gram_jacobi<T>(Jl, ldj, rows, nc, Vl, ldv, nc, fro2, stop, JACOBI_MAX_SWEEPS, NW, lds);
+        } else {
+            __syncthreads();
+            sweeps = wg_gram_jacobi<T>(Jl, ldj, rows, nc, w.v1, nc, nc, fro2, stop, JACOBI_MAX_SWEEPS, NW, lds);
+        }
+        __syncthreads();
+        for (ColWalk p(threadIdx.x, JW_THREADS, rows); p.c < nc; p.next())
+            w.j[p.i + (int64_t) p.c * rows] = Jl[p.i + p.c * ldj];
+        if (vin)
+            for (ColWalk p(threadIdx.x, JW_THREADS, nc); p.c < nc; p.next())
+                w.v1[p.i + (int64_t) p.c * nc] = Vl[p.i + p.c * ldv];
     } else {
-        bI = (step + bp) % (nbp - 1);
-        bJ = (step - bp + nbp - 1) % (nbp - 1);
+        sweeps = wg_gram_jacobi<T>(w.j, rows, rows, nc, w.v1, nc, nc, fro2, stop, JACOBI_MAX_SWEEPS, NW, lds);
     }
-    if (bI > bJ) {
-        const int t = bI;
-        bI = bJ;
-        bJ = t;
+    if (threadIdx.x == 0) w.hdr[HDR_SWEEPS] = sweeps;
+}
+
+// What the steps of one multi-workgroup Jacobi work on.  The host knows the core's width and norm by
+// then, so a step starts on its columns at once instead of after two dependent reads of the header (7.2 ->
+// 6.6 us per step of a 128-column core).  rec: the records of two launches (npair each, alternating),
+// then their flags; they sit in the core-QR region of the workspace (j2 and what follows), which the
+// plain form does not use otherwise.
+template <typename T>
+struct MwJacobi {
+    T *j, *v, *rec;
+    int32_t *flags;
+    int rows, ncols, nbp;  // nbp: blocks, rounded up to even
+    T fro2;
+};
+
+// Step `step` of sweep `sweep` (blockIdx.y 0), and V's part of the step before it (blockIdx.y >= 1);
+// `last`: only V's part, after the last step launched.  GROUPS: 16-row groups per wave.
+template <typename T, int GROUPS>
+__global__ void __launch_bounds__(MW_WAVES *WAVE) k_jacobi_step(MwJacobi<T> m, int sweep, int step, int last) {
+    __shared__ T lds[MW_LDS];
+    const int npair = m.nbp / 2, steps = m.nbp - 1;
+    const bool rotate = blockIdx.y == 0;
+    int launch = sweep * steps + step;  // the launch whose pair this workgroup works on
+    if (rotate) {
+        if (last) return;
+    } else {
+        if (launch == 0) return;
+        --launch;
     }
-    if (bI * B >= ncols) return;
-    const T fro2 = (T) __longlong_as_double(w.hdr[HDR_JFRO2]);
-    const T floor2 = Eps<T>::value * Eps<T>::value * fro2;
-    const T tol = sqrt(T(rows)) * Eps<T>::value;
-    const int any = coop_jacobi_tile_rec<T, RPL, MW_TW>(w.j, rows, ncols, rows, w.v1, ncols, bI * B, bJ * B,
-                                                         step == 0, tol, floor2, lds);
-    if ((any & JROT_LARGE) && threadIdx.x == 0) flags[sweep] = 1;
+    const int sw = launch / steps, st = launch % steps, bp = (int) blockIdx.x;
+    int cI, cJ;
+    if (!jacobi_pair_cols(bp, st, m.nbp, GJ_B, m.ncols, cI, cJ)) return;
+    if (st > 0 && cJ >= m.ncols) return;
+    const int32_t live = sw > 0 ? m.flags[sw - 1] : 1;  // 0: converged in an earlier sweep
+    T *rec = m.rec + (int64_t) ((launch & 1) * npair + bp) * MW_REC;
+    int32_t *used = reinterpret_cast<int32_t *>(m.rec + (int64_t) 2 * npair * MW_REC) + (launch & 1) * npair + bp;
+    if (rotate) {
+        const GramTol<T> g(m.fro2, m.rows, JacobiStopCos<T>::tight);
+        const int any =
+                mw_rotate_tile<T, GROUPS>(m.j, m.rows, m.ncols, cI, cJ, st == 0, live != 0, g, rec, used, lds);
+        if ((any & JROT_LARGE) && threadIdx.x == 0) m.flags[sw] = 1;
+    } else if (live && *used) {
+        mw_apply_v<T>(m.v, m.ncols, m.ncols, cI, cJ, rec, ((int) blockIdx.y - 1) * MW_VROWS);
+    }
 }
 
 template <typename T>
+static void launch_jacobi_step(hipStream_t s, const MwJacobi<T> &m, int sweep, int step, int last) {
+    const dim3 wg(MW_WAVES * WAVE), grid(m.nbp / 2, 1 + (m.ncols + MW_VROWS - 1) / MW_VROWS);
+    const int groups = (m.rows + 16 * MW_WAVES - 1) / (16 * MW_WAVES);
+    if (groups <= 1) hipLaunchKernelGGL((k_jacobi_step<T, 1>), grid, wg, 0, s, m, sweep, step, last);
+    else if (groups <= 2) hipLaunchKernelGGL((k_jacobi_step<T, 2>), grid, wg, 0, s, m, sweep, step, last);
+    else if (groups <= 4) hipLaunchKernelGGL((k_jacobi_step<T, 4>), grid, wg, 0, s, m, sweep, step, last);
+    else hipLaunchKernelGGL((k_jacobi_step<T, 6>), grid, wg, 0, s, m, sweep, step, last);
+}
+static_assert(JACOBI_ROWS_MAX <= 16 * MW_WAVES * 6, "the widest k_jacobi_step holds the tallest core");
+
+// `launched` sweeps of the multi-workgroup Jacobi, or -1 after the one-workgroup one.
+template <typename T>
 __global__ void HCAMD_KERNEL k_svd_finish(RecompDesc<T> d, const int32_t *flags, int launched) {
-    int sweeps = launched;
+    Ws<T> w = ws_of(d);
+    int sweeps = launched < 0 ? (int) w.hdr[HDR_SWEEPS] : launched;
     for (int s = 0; s < launched; ++s)
         if (flags[s] == 0) {
             sweeps = s;
@@ -273,42 +333,53 @@ __global__ void HCAMD_KERNEL k_svd_finish(RecompDesc<T> d, const int32_t *flags,
     ph_svd_finish<T>(d, sweeps);
 }
 
-template <typename T, int RPL>
-static void launch_jacobi_sweep(hipStream_t s, const RecompDesc<T> &d, int32_t *flags, int sweep, int steps,
-                                int grid) {
-    for (int st = 0; st < steps; ++st)
-        hipLaunchKernelGGL((k_jacobi_step<T, RPL>), dim3(grid), dim3(NT), 0, s, d, flags, sweep, st);
-}
-
-// Core SVD over many workgroups: core build, Jacobi sweeps launched in chunks (the host reads the
-// last sweep's flag between chunks, through the pinned word `host_flag`), then the rank rule.
+// The whole core SVD.  Cores that may be wide (kk columns are known here) have their width read back
+// once, so that the steps are launched for the columns there are: the core is cut at the rounding
+// level, often at half of kk, and a launch that finds nothing to do costs as much as a tenth of a step.
+// The sweeps are launched in chunks; the host reads the last sweep's flag between chunks.
 template <typename T>
-static hipError_t launch_core_svd_mw(hipStream_t s, const RecompDesc<T> &d, int mu, int kk, int32_t *flags,
-                                     volatile int32_t *host_flag) {
+static hipError_t launch_core_svd(hipStream_t s, const RecompDesc<T> &d, int mu, int kk, int32_t *flags,
+                                  volatile int64_t *host) {
     hipLaunchKernelGGL(k_core<T>, dim3(1), dim3(NT), 0, s, d, flags);
-    constexpr int B = MW_TW / 2;
-    const int nblk = (kk + B - 1) / B;
-    const int nbp = nblk + (nblk & 1);
-    const int steps = nbp - 1, grid = nbp / 2;
-    const int rpl = (mu + NT - 1) / NT;
-    int launched = 0, chunk = 6;
+    hipError_t e;
+    int kt = kk;
+    T fro2 = T(0);
+    if (kk >= MW_MIN_COLS) {
+        static_assert(HDR_JFRO2 == HDR_KT + 1, "read together");
+        const int64_t *hdr = reinterpret_cast<const int64_t *>(d.ws);
+        e = hipMemcpyAsync((void *) host, hdr + HDR_KT, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return e;
+        kt = (int) host[0];
+        const int64_t bits = host[1];
+        double f;
+        memcpy(&f, &bits, sizeof(f));
+        fro2 = (T) f;
+    }
+    if (kt < MW_MIN_COLS) {
+        hipLaunchKernelGGL(k_jacobi_wg<T>, dim3(1), dim3(JW_THREADS), JW_LDS_BYTES, s, d);
+        hipLaunchKernelGGL(k_svd_finish<T>, dim3(1), dim3(NT), 0, s, d, flags, -1);
+        return hipGetLastError();
+    }
+    const WsLayout L = ws_layout<T>(d.m, d.n, d.kmax, d.max_rank);
+    const int nblk = (kt + GJ_B - 1) / GJ_B, nbp = nblk + (nblk & 1);
+    const MwJacobi<T> m{d.ws + L.j, d.ws + L.v1, d.ws + L.j2, flags, mu, kt, nbp, fro2};
+    // most cores converge within 5 to 8 sweeps: the first five are launched at once, then one at a time
+    int launched = 0, chunk = 5;
     while (launched < JACOBI_MAX_SWEEPS) {
         const int end = launched + chunk < JACOBI_MAX_SWEEPS ? launched + chunk : JACOBI_MAX_SWEEPS;
-        for (int sw = launched; sw < end; ++sw) {
-            if (rpl <= 1) launch_jacobi_sweep<T, 1>(s, d, flags, sw, steps, grid);
-            else if (rpl == 2) launch_jacobi_sweep<T, 2>(s, d, flags, sw, steps, grid);
-            else launch_jacobi_sweep<T, 3>(s, d, flags, sw, steps, grid);
-        }
+        for (int sw = launched; sw < end; ++sw)
+            for (int st = 0; st < nbp - 1; ++st) launch_jacobi_step<T>(s, m, sw, st, 0);
         launched = end;
-        hipError_t e = hipGetLastError();
+        e = hipGetLastError();
+        if (e == hipSuccess)
+            e = hipMemcpyAsync((void *) host, flags + launched - 1, sizeof(int32_t), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) return e;
-        e = hipMemcpyAsync((void *) host_flag, flags + launched - 1, sizeof(int32_t), hipMemcpyDeviceToHost, s);
-        if (e != hipSuccess) return e;
-        e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return e;
-        if (*host_flag == 0) break;
-        chunk = 2;
+        if (*reinterpret_cast<volatile int32_t *>(host) == 0) break;
+        chunk = 1;
     }
+    launch_jacobi_step<T>(s, m, launched, 0, 1);
     hipLaunchKernelGGL(k_svd_finish<T>, dim3(1), dim3(NT), 0, s, d, flags, launched);
     return hipGetLastError();
 }
@@ -456,7 +527,7 @@ __global__ void HCAMD_KERNEL k_batched(const BatchEntry<T> *entries, const int32
             ph_core_build<T, false>(d);
             ph_core_qr<T, PB>(d, lds);
             t_qry = HCAMD_TSTAMP();
-            ph_svd_nov<T>(d, lds);
+            ph_svd_nov<T>(d);
             __syncthreads();
             t_svd = HCAMD_TSTAMP();
         }
@@ -563,23 +634,20 @@ static int clamp_grid(int64_t work) {
 
 template <typename T>
 hipError_t launch_recomp_pre(hipStream_t s, const RecompDesc<T> &d, int64_t K, int64_t lds_bytes, int pb,
-                             int32_t *jflags, int32_t *host_flag, T *vpan) {
+                             int32_t *jflags, int64_t *host, T *vpan) {
     const int64_t m = d.m, n = d.n;
     const int64_t mu = m < K ? m : K;
     const int64_t kk = n < mu ? n : mu;
     hipLaunchKernelGGL(k_stack<T>, dim3(clamp_grid(m * K)), dim3(NT), 0, s, d);
-    hipError_t e = (vpan && K >= MW_MIN_QR_COLS) ? launch_qr_mw<T>(s, d, lds_bytes, pb, 0, (int) m, (int) K, vpan)
+    hipError_t e = (K >= MW_MIN_QR_COLS) ? launch_qr_mw<T>(s, d, lds_bytes, pb, 0, (int) m, (int) K, vpan)
                                                  : launch_qr<T>(s, d, lds_bytes, pb, 0);
     if (e != hipSuccess) return e;
     const int ytiles = (int) (((n + GT_M - 1) / GT_M) * ((mu + GT_N - 1) / GT_N));
     hipLaunchKernelGGL(k_y<T>, dim3(ytiles), dim3(NT), 0, s, d);
-    e = (vpan && mu >= MW_MIN_QR_COLS) ? launch_qr_mw<T>(s, d, lds_bytes, pb, 1, (int) n, (int) mu, vpan)
+    e = (mu >= MW_MIN_QR_COLS) ? launch_qr_mw<T>(s, d, lds_bytes, pb, 1, (int) n, (int) mu, vpan)
                                        : launch_qr<T>(s, d, lds_bytes, pb, 1);
     if (e != hipSuccess) return e;
-    if (jflags && host_flag && kk >= MW_MIN_COLS && mu <= JACOBI_ROWS_MAX)
-        return launch_core_svd_mw<T>(s, d, (int) mu, (int) kk, jflags, host_flag);
-    hipLaunchKernelGGL(k_svd<T>, dim3(1), dim3(NT), 0, s, d);
-    return hipGetLastError();
+    return launch_core_svd<T>(s, d, (int) mu, (int) kk, jflags, host);
 }
 
 template <typename T>
@@ -647,14 +715,15 @@ hipError_t set_kernel_lds_limits(int64_t lds_bytes) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds_bytes);
         if (e != hipSuccess) return e;
     }
-    return hipSuccess;
+    return hipFuncSetAttribute((const void *) k_jacobi_wg<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int) JW_LDS_BYTES);
 }
 
 #define HCAMD_INSTANTIATE(T)                                                                                     \
     template hipError_t launch_gemm<T>(hipStream_t, int, int, int, T, const T *, int64_t, bool, const T *,      \
                                        int64_t, bool, T, T *, int64_t);                                          \
     template hipError_t launch_recomp_pre<T>(hipStream_t, const RecompDesc<T> &, int64_t, int64_t, int, int32_t *, \
-                                             int32_t *, T *);                                                    \
+                                             int64_t *, T *);                                                    \
     template hipError_t launch_recomp_post<T>(hipStream_t, const RecompDesc<T> &, int64_t, int64_t, int);        \
     template hipError_t launch_readjust_ddc<T>(hipStream_t, const T *, int64_t, int64_t, T *);                   \
     template hipError_t launch_fill_identity<T>(hipStream_t, T *, int64_t);                                      \

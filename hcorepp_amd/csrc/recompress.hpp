@@ -1179,61 +1179,9 @@ __device__ void ph_core_qr(const RecompDesc<T> &d, T *lds) {
 // ---------------------------------------------------------------------------
 // Phase: Jacobi + sigma + sort + rank (single workgroup).
 // ---------------------------------------------------------------------------
-template <typename T, int RPL, int RPLV, int TW>
-__device__ HCAMD_PHASE_ATTR int block_jacobi_nl(T *J, int rows, int ncols, T *V, T *gbuf) {
-    return wg_block_jacobi<T, RPL, RPLV, TW>(J, rows, ncols, rows, V, ncols, JACOBI_MAX_SWEEPS, gbuf);
-}
-
-template <typename T, int RPL, int RPLV, int TW>
-__device__ HCAMD_PHASE_ATTR int coop_jacobi_nl(T *J, int rows, int ncols, T *V, T *gbuf) {
-    return wg_coop_jacobi<T, RPL, RPLV, TW>(J, rows, ncols, rows, V, ncols, JACOBI_MAX_SWEEPS, gbuf);
-}
-
-// Tile shape by core rows and (truncated) width.  Per-wave tiles (a wave owns a whole tile of J
-// and V columns; four tiles in flight per workgroup) with shapes that fit 256 VGPRs without
-// spilling; for 193-256 rows the four waves share 16-column tiles instead (rows split across
-// waves, one barrier per rotation round), which measured faster there because it needs half the
-// passes over J and V of the widest per-wave tile that fits.  `exact_core` (a core sized at the
-// rounding level only) also takes the shared tiles for 129-192 rows: 7 % faster on the nb=512
-// benchmark batch, while cores cut by a rank tolerance ran 8 % slower with them.
-template <typename T>
-__device__ int run_block_jacobi(T *J, int rows, int ncols, T *V, T *gbuf, bool exact_core) {
-    if (rows <= 64) return block_jacobi_nl<T, 1, 1, 16>(J, rows, ncols, V, gbuf);
-    if (rows <= 128)
-        return ncols <= 64 ? block_jacobi_nl<T, 2, 1, 8>(J, rows, ncols, V, gbuf)
-                           : block_jacobi_nl<T, 2, 2, 8>(J, rows, ncols, V, gbuf);
-    if (rows <= 192) {
-        if (exact_core) return coop_jacobi_nl<T, 1, 1, 16>(J, rows, ncols, V, gbuf);
-        return ncols <= 128 ? block_jacobi_nl<T, 3, 2, 8>(J, rows, ncols, V, gbuf)
-                            : block_jacobi_nl<T, 3, 3, 4>(J, rows, ncols, V, gbuf);
-    }
-    if (rows <= 256) return coop_jacobi_nl<T, 1, 1, 16>(J, rows, ncols, V, gbuf);
-    if (rows <= 320)
-        return ncols <= 192 ? block_jacobi_nl<T, 5, 3, 4>(J, rows, ncols, V, gbuf)
-                            : block_jacobi_nl<T, 5, 5, 4>(J, rows, ncols, V, gbuf);
-    if (rows <= 384) {
-        if (ncols <= 192) return block_jacobi_nl<T, 6, 3, 4>(J, rows, ncols, V, gbuf);
-        if (ncols <= 256) return block_jacobi_nl<T, 6, 4, 4>(J, rows, ncols, V, gbuf);
-        return block_jacobi_nl<T, 6, 6, 4>(J, rows, ncols, V, gbuf);
-    }
-    if (rows <= 512)
-        return ncols <= 256 ? block_jacobi_nl<T, 8, 4, 4>(J, rows, ncols, V, gbuf)
-                            : block_jacobi_nl<T, 8, 8, 2>(J, rows, ncols, V, gbuf);
-    if (rows <= 640)
-        return ncols <= 320 ? block_jacobi_nl<T, 10, 5, 2>(J, rows, ncols, V, gbuf)
-                            : block_jacobi_nl<T, 10, 10, 2>(J, rows, ncols, V, gbuf);
-    return ncols <= 384 ? block_jacobi_nl<T, 12, 6, 2>(J, rows, ncols, V, gbuf)
-                        : block_jacobi_nl<T, 12, 12, 2>(J, rows, ncols, V, gbuf);
-}
-
 constexpr int JACOBI_ROWS_MAX = 768;
-// LDS of the core-SVD phase: ph_core's row norms (<= JACOBI_ROWS_MAX + NWAVES) and the block Jacobi's
-// reduction slots, which reuse the same space.
-constexpr int JACOBI_LDS_ELEMS = JACOBI_ROWS_MAX + NWAVES + 8;
-static_assert(JACOBI_LDS_ELEMS >= block_jacobi_lds_elems<double, 16>() &&
-                      JACOBI_LDS_ELEMS >= coop_jacobi_lds_elems<double, 16>(),
-              "core-SVD LDS covers both Jacobi variants");
-static_assert(JACOBI_LDS_ELEMS >= JACOBI_ROWS_MAX + NWAVES, "ph_core scratch must fit the core-SVD LDS");
+// LDS of the core set-up: ph_core_size's row norms and threshold.
+constexpr int CORE_LDS_ELEMS = JACOBI_ROWS_MAX + NWAVES + 8;
 
 // Tail of the core SVD once the Jacobi has converged (`sweeps` used): singular values, their
 // descending order, the rank rule and the header words.
@@ -1309,107 +1257,80 @@ __device__ void ph_svd_finish(const RecompDesc<T> &d, int sweeps) {
     __syncthreads();
 }
 
-template <typename T>
-__device__ void ph_svd(const RecompDesc<T> &d, T *lds) {
-    Ws<T> w = ws_of(d);
-    const Dims z = dims_of(d, w);
-    int sweeps = 0;
-    if (z.mu > JACOBI_ROWS_MAX) {
-        if (threadIdx.x == 0) w.hdr[HDR_STATUS] |= STATUS_TOO_BIG;
-    } else {
-        HCAMD_SUB_BEGIN(t_jac);
-        const bool exact_core = !d.rank_model && !(d.model_tol > 0.0);
-        if (w.hdr[HDR_CQR]) sweeps = run_block_jacobi<T>(w.j2, z.kt, z.kt, w.v1, lds, exact_core);
-        else sweeps = run_block_jacobi<T>(w.j, z.mu, z.kt, w.v1, lds, exact_core);
-        HCAMD_SUB_END(t_jac, w.hdr, 3);
-#ifdef HCAMD_PHASE_TIMING
-        if (threadIdx.x == 0) w.hdr[HDR_SUB + 7] = sweeps + 1000 * z.kt;  // timing build: sweeps and core width
-#endif
-    }
-    ph_svd_finish<T>(d, sweeps);
-}
-
 // ---------------------------------------------------------------------------
 // Batched form: the core Jacobi without V.  The rotations only orthogonalise the columns of the
 // core X (X V1 = Z); the right factor is recovered afterwards from the left one: X = Z V1^T
-// gives X^T U = V1 Sigma for U = Z Sigma^-1 (ph_recon_nov).  Dropping V halves the Jacobi's data
-// and frees the registers that let the tiles double their width (half the passes over X per
-// sweep).  A core of at most BATCH_LDS_BYTES / sizeof(T) - NOV_GBUF elements is moved into the
-// kernel's dynamic LDS for the whole iteration, so its sweeps read no global memory.
+// gives X^T U = V1 Sigma for U = Z Sigma^-1 (ph_recon_nov), which halves the Jacobi's data.
+// The core moves into the kernel's dynamic LDS for the whole iteration where it fits with the waves'
+// tile matrices (up to 93 square columns), so that its sweeps read no global memory; wider cores pass
+// through it by super-blocks (wg_staged_jacobi), the waves sharing tiles where the LDS holds fewer
+// than four at a time (32 columns per super-block up to 138 rows, 16 up to 276, 8 up to 554); taller
+// ones are rotated in global memory.
 // ---------------------------------------------------------------------------
 constexpr int64_t BATCH_LDS_BYTES = 78 * 1024;  // dynamic LDS per workgroup of the batched kernel
-constexpr int NOV_GBUF = 16;                     // reduction slots ahead of the LDS-resident core
-static_assert(NOV_GBUF >= block_jacobi_lds_elems<double, 16>(), "the block Jacobi's slots fit before the core");
 
 template <typename T>
 __host__ __device__ constexpr int64_t nov_lds_cap() {
-    return BATCH_LDS_BYTES / (int64_t) sizeof(T) - NOV_GBUF;
+    return BATCH_LDS_BYTES / (int64_t) sizeof(T) - gram_jacobi_lds<T>(NWAVES);
 }
 
-// LDS-resident core: J (rows x ncols, ld rows) at element NOV_GBUF of the dynamic LDS, the
-// reduction slots before it.  The pointers are formed here from the dynamic LDS symbol so that
+// The LDS pointers of the variants below are formed from the dynamic LDS symbol inside them, so that
 // every access of the iteration is an LDS instruction.
-template <typename T, int RPL, int TW>
-__device__ HCAMD_PHASE_ATTR int jacobi_nov_lds_nl(int rows, int ncols) {
-    extern __shared__ unsigned char smem_raw[];
-    T *gbuf = reinterpret_cast<T *>(smem_raw);
-    return wg_block_jacobi<T, RPL, 0, TW>(gbuf + NOV_GBUF, rows, ncols, rows, nullptr, 0, JACOBI_MAX_SWEEPS, gbuf);
-}
-
-// Core in global memory: for up to 128 rows the next tile is loaded while the current one
-// rotates (measured on the benchmark batch: 6 % less Jacobi time for 100-128-column cores;
-// slower for taller tiles, whose two register tiles no longer fit without spills).
-template <typename T, int RPL, int TW>
-__device__ HCAMD_PHASE_ATTR int jacobi_nov_nl(T *J, int rows, int ncols, T *gbuf) {
-    return wg_block_jacobi<T, RPL, 0, TW, (RPL <= 2)>(J, rows, ncols, rows, nullptr, 0, JACOBI_MAX_SWEEPS, gbuf);
-}
-
-// Core in global memory staged through LDS by super-blocks of W columns (wg_staged_jacobi): the
-// buffer after the reduction slots holds two super-blocks.
-template <typename T, int RPL, int TW>
-__device__ HCAMD_PHASE_ATTR int jacobi_nov_staged_nl(T *J, int rows, int ncols, int W) {
-    extern __shared__ unsigned char smem_raw[];
-    T *gbuf = reinterpret_cast<T *>(smem_raw);
-    return wg_staged_jacobi<T, RPL, TW>(J, rows, ncols, gbuf + NOV_GBUF, W, JACOBI_MAX_SWEEPS, gbuf);
-}
-
-template <typename T, int RPL, int TW>
-__device__ int jacobi_nov_shape(T *J, int rows, int ncols, T *lds, bool resident) {
-    if (resident) return jacobi_nov_lds_nl<T, RPL, TW>(rows, ncols);
-    const int W = staged_width(rows, TW / 2, nov_lds_cap<T>());
-    return W > 0 ? jacobi_nov_staged_nl<T, RPL, TW>(J, rows, ncols, W) : jacobi_nov_nl<T, RPL, TW>(J, rows, ncols, lds);
-}
-
-// One-sided Jacobi of J (rows x ncols, ld rows) in place, without V; `lds` is the kernel's
-// dynamic LDS (BATCH_LDS_BYTES).  Returns the sweeps used.
 template <typename T>
-__device__ int run_jacobi_nov(T *J, int rows, int ncols, T *lds) {
-    const int64_t ne = (int64_t) rows * ncols;
-    const bool resident = ne <= nov_lds_cap<T>();
-    T *Jl = lds + NOV_GBUF;
-    if (resident) {
-        wg_copy(Jl, J, ne);
-        __syncthreads();
+__device__ HCAMD_PHASE_ATTR int jacobi_nov_lds(T *J, int rows, int ncols) {
+    extern __shared__ unsigned char smem_raw[];
+    T *lds = reinterpret_cast<T *>(smem_raw);
+    T *Jl = lds + gram_jacobi_lds<T>(NWAVES);
+    const int ld = rows | 1;
+    T part = T(0);
+    for (ColWalk p(threadIdx.x, NT, rows); p.c < ncols; p.next()) {
+        const T a = J[p.i + (int64_t) p.c * rows];
+        Jl[p.i + p.c * ld] = a;
+        part += a * a;
     }
-    int sweeps;
-    if (rows <= 64) sweeps = jacobi_nov_shape<T, 1, 16>(J, rows, ncols, lds, resident);
-    else if (rows <= 128) sweeps = jacobi_nov_shape<T, 2, 16>(J, rows, ncols, lds, resident);
-    else if (rows <= 192) sweeps = jacobi_nov_shape<T, 3, 8>(J, rows, ncols, lds, resident);
-    else if (rows <= 256) sweeps = jacobi_nov_shape<T, 4, 8>(J, rows, ncols, lds, resident);
-    else if (rows <= 384) sweeps = jacobi_nov_shape<T, 6, 8>(J, rows, ncols, lds, resident);
-    else if (rows <= 512) sweeps = jacobi_nov_shape<T, 8, 4>(J, rows, ncols, lds, resident);
-    else sweeps = jacobi_nov_shape<T, 12, 4>(J, rows, ncols, lds, resident);
-    if (resident) {
-        __syncthreads();
-        wg_copy(J, Jl, ne);
-        __syncthreads();
-    }
+    const T fro2 = wg_sum(part, lds);
+    const int sweeps = wg_gram_jacobi<T>(Jl, ld, rows, ncols, nullptr, 0, 0, fro2, JacobiStopCos<T>::loose,
+                                         JACOBI_MAX_SWEEPS, NWAVES, lds);
+    __syncthreads();
+    for (ColWalk p(threadIdx.x, NT, rows); p.c < ncols; p.next()) J[p.i + (int64_t) p.c * rows] = Jl[p.i + p.c * ld];
+    __syncthreads();
     return sweeps;
+}
+
+template <typename T, int NS>
+__device__ HCAMD_PHASE_ATTR int jacobi_nov_staged(T *J, int rows, int ncols) {
+    extern __shared__ unsigned char smem_raw[];
+    T *lds = reinterpret_cast<T *>(smem_raw);
+    return wg_staged_jacobi<T, NS>(J, rows, ncols, lds + gram_jacobi_lds<T>(NWAVES), JacobiStopCos<T>::loose,
+                                   JACOBI_MAX_SWEEPS, lds);
+}
+
+template <typename T>
+__device__ HCAMD_PHASE_ATTR int jacobi_nov_global(T *J, int rows, int ncols) {
+    extern __shared__ unsigned char smem_raw[];
+    T *lds = reinterpret_cast<T *>(smem_raw);
+    T part = T(0);
+    for (int64_t e = threadIdx.x; e < (int64_t) rows * ncols; e += NT) part += J[e] * J[e];
+    const T fro2 = wg_sum(part, lds);
+    return wg_gram_jacobi<T>(J, rows, rows, ncols, nullptr, 0, 0, fro2, JacobiStopCos<T>::loose, JACOBI_MAX_SWEEPS,
+                             NWAVES, lds);
+}
+
+// One-sided Jacobi of J (rows x ncols, ld rows) in place, without V, in the kernel's dynamic LDS
+// (BATCH_LDS_BYTES).  Returns the sweeps used.
+template <typename T>
+__device__ int run_jacobi_nov(T *J, int rows, int ncols) {
+    const int64_t cap = nov_lds_cap<T>(), ld = rows | 1;
+    if (ld * ncols <= cap) return jacobi_nov_lds<T>(J, rows, ncols);
+    if (ld * (2 * GJ_B * NWAVES) <= cap) return jacobi_nov_staged<T, 1>(J, rows, ncols);
+    if (ld * (GJ_B * NWAVES) <= cap) return jacobi_nov_staged<T, 2>(J, rows, ncols);
+    if (ld * (GJ_B * NWAVES / 2) <= cap) return jacobi_nov_staged<T, 4>(J, rows, ncols);
+    return jacobi_nov_global<T>(J, rows, ncols);
 }
 
 // Core SVD of the batched form: the Jacobi without V, then sigma, order and rank (ph_svd_finish).
 template <typename T>
-__device__ void ph_svd_nov(const RecompDesc<T> &d, T *lds) {
+__device__ void ph_svd_nov(const RecompDesc<T> &d) {
     Ws<T> w = ws_of(d);
     const Dims z = dims_of(d, w);
     int sweeps = 0;
@@ -1417,8 +1338,8 @@ __device__ void ph_svd_nov(const RecompDesc<T> &d, T *lds) {
         if (threadIdx.x == 0) w.hdr[HDR_STATUS] |= STATUS_TOO_BIG;
     } else {
         HCAMD_SUB_BEGIN(t_jac);
-        if (w.hdr[HDR_CQR]) sweeps = run_jacobi_nov<T>(w.j2, z.kt, z.kt, lds);
-        else sweeps = run_jacobi_nov<T>(w.j, z.mu, z.kt, lds);
+        if (w.hdr[HDR_CQR]) sweeps = run_jacobi_nov<T>(w.j2, z.kt, z.kt);
+        else sweeps = run_jacobi_nov<T>(w.j, z.mu, z.kt);
         HCAMD_SUB_END(t_jac, w.hdr, 3);
 #ifdef HCAMD_PHASE_TIMING
         if (threadIdx.x == 0) w.hdr[HDR_SUB + 7] = sweeps + 1000 * z.kt;  // timing build: sweeps and core width
