@@ -77,10 +77,13 @@ hcorepp_status ensure_lds_limits() {
     std::lock_guard<std::mutex> lk(g_lds_mutex);
     if (!g_lds_ready_d) {
         HIP_TRY(set_kernel_lds_limits<double>(kLdsBytes));
+        HIP_TRY(set_tileops_lds_limits<double>());
+        HIP_TRY(set_cholesky_lds_limits());
         g_lds_ready_d = true;
     }
     if (!g_lds_ready_s) {
         HIP_TRY(set_kernel_lds_limits<float>(kLdsBytes));
+        HIP_TRY(set_tileops_lds_limits<float>());
         g_lds_ready_s = true;
     }
     return HCOREPP_OK;
@@ -1304,18 +1307,20 @@ hcorepp_status hcorepp_trsm_batch_d(hcorepp_ctx *ctx, int64_t n, const hcorepp_t
     if ((st = validate_tile<double>(L, "L"))) return st;
     if (L->type != HCOREPP_DENSE || L->rows != L->cols) return fail(HCOREPP_ERR_INVALID, "L must be square dense");
     std::vector<CholTrsm> jobs;
+    int64_t max_rank = 0;
     for (int64_t i = 0; i < n; ++i) {
         if ((st = validate_tile<double>(&B[i], "B[i]"))) return st;
         if (B[i].type != HCOREPP_COMPRESSED || B[i].cols != L->rows)
             return fail(HCOREPP_ERR_INVALID, "trsm: B[%lld] must be compressed with cols == L rows", (long long) i);
         if (B[i].rank == 0) continue;
+        max_rank = std::max(max_rank, B[i].rank);
         jobs.push_back(CholTrsm{(double *) B[i].data + B[i].rows * B[i].max_rank, (const double *) L->data,
                                 B[i].rank, L->rows, L->ld});
     }
     if ((st = arena_begin(ctx, sizeof(CholTrsm) * (jobs.size() + 1) + 4096))) return st;
     CholTrsm *dj;
     if ((st = upload_jobs(ctx, jobs, &dj))) return st;
-    HIP_TRY(launch_trsm_v(ctx->stream, dj, (int) jobs.size()));
+    HIP_TRY(launch_trsm_v(ctx->stream, dj, (int) jobs.size(), (int) max_rank, (int) L->rows));
     return HCOREPP_OK;
 }
 

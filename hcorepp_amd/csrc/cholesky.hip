@@ -9,6 +9,7 @@
 // tile; potrf is blocked over several launches.
 #include "kernels.hpp"
 #include "cholesky.hpp"
+#include "trsm.hpp"
 
 namespace hcamd {
 
@@ -129,11 +130,16 @@ __global__ void k_zero_int(int *p) {
     if (threadIdx.x == 0) *p = 0;
 }
 
-// V (r x n, ld r) <- V L^{-T} for lower-triangular L (n x n, ld ldl): one workgroup per tile.
+// V (r x n, ld r) <- V L^{-T} for lower-triangular L (n x n, ld ldl): the rows of V solve L x^T = v^T,
+// 16 rows of one tile per workgroup.  (One workgroup per tile with a row per thread took 358 us for tiles
+// of 256 columns.)
 __global__ void HCAMD_KERNEL k_trsm_v(const CholTrsm *jobs) {
-    __shared__ double lds[ROWS_TRSM_LDS];
-    const CholTrsm jb = jobs[blockIdx.x];
-    rows_trsm_lt<double>(jb.v, (int) jb.rank, (int) jb.n, jb.rank, jb.l, jb.ldl, lds);
+    extern __shared__ unsigned char smem_raw[];
+    const CholTrsm jb = jobs[blockIdx.y];
+    const int r0 = (int) blockIdx.x * TS_NV, left = (int) jb.rank - r0;
+    if (left <= 0) return;
+    wg_trsm<double>(jb.v + r0, jb.rank, 1, left < TS_NV ? left : TS_NV, (int) jb.n, jb.l, jb.ldl, false, true, false,
+                    1.0, reinterpret_cast<double *>(smem_raw));
 }
 
 // A (n x n dense) <- A - U (V V^T) U^T, with scratch W (r x r) and T (n x r); the strict upper
@@ -198,9 +204,18 @@ hipError_t launch_potrf(hipStream_t s, T *A, int n, int64_t lda, int *info) {
 }
 template hipError_t launch_potrf<double>(hipStream_t, double *, int, int64_t, int *);
 template hipError_t launch_potrf<float>(hipStream_t, float *, int, int64_t, int *);
-hipError_t launch_trsm_v(hipStream_t s, const CholTrsm *jobs, int n) {
-    if (n > 0) hipLaunchKernelGGL(k_trsm_v, dim3(n), dim3(NT), 0, s, jobs);
+hipError_t launch_trsm_v(hipStream_t s, const CholTrsm *jobs, int n, int max_rank, int len) {
+    // jobs along y (at most 65535 per launch)
+    for (int j0 = 0; j0 < n; j0 += 65535) {
+        const int nj = n - j0 < 65535 ? n - j0 : 65535;
+        hipLaunchKernelGGL(k_trsm_v, dim3((max_rank + TS_NV - 1) / TS_NV, nj), dim3(NT), (size_t) ts_lds_bytes<double>(len),
+                           s, jobs + j0);
+    }
     return hipGetLastError();
+}
+hipError_t set_cholesky_lds_limits() {
+    return hipFuncSetAttribute((const void *) k_trsm_v, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int) ts_lds_bytes<double>(ts_len_lds<double>()));
 }
 hipError_t launch_syrk(hipStream_t s, const CholSyrk *jobs, int n) {
     if (n > 0) hipLaunchKernelGGL(k_syrk, dim3(n), dim3(NT), 0, s, jobs);

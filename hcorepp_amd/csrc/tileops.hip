@@ -13,6 +13,7 @@
 #include "kernels.hpp"
 #include "cholesky.hpp"
 #include "tileops.hpp"
+#include "trsm.hpp"
 
 namespace hcamd {
 
@@ -50,34 +51,20 @@ __global__ void HCAMD_KERNEL k_lower_to_tri(const T *W, int n, T *A, int64_t lda
     }
 }
 
-// Triangular solves with many right-hand sides, one thread per independent vector: for side
+// Triangular solves with many right-hand sides, 16 independent vectors per workgroup (wg_trsm): for side
 // Left the columns of B (m x n) solve op(A) x = alpha b (A m x m); for side Right the rows solve
 // x op(A) = alpha b, i.e. op(A)^T x^T = alpha b^T (A n x n).  M = op(A) or op(A)^T is lower or
 // upper, forward or back substitution accordingly; unit diagonals are not read.
 template <typename T>
 __global__ void HCAMD_KERNEL k_trsm_vec(int m, int n, T alpha, const T *A, int64_t lda, T *B, int64_t ldb, int left,
                                         int upper, int trans, int unit) {
+    extern __shared__ unsigned char smem_raw[];
     const int len = left ? m : n, count = left ? n : m;
-    const int v = (int) (blockIdx.x * NT + threadIdx.x);
-    if (v >= count) return;
-    const int64_t estride = left ? 1 : ldb;            // stride between elements of one vector
-    T *x = B + (left ? (int64_t) v * ldb : (int64_t) v);
-    const bool teff = left ? trans != 0 : trans == 0;  // M(i, j) = A(j, i) when set
-    const bool lower = (upper == 0) != teff;
-    auto M = [&](int i, int j) -> T { return teff ? A[j + (int64_t) i * lda] : A[i + (int64_t) j * lda]; };
-    if (lower) {
-        for (int i = 0; i < len; ++i) {
-            T s = alpha * x[i * estride];
-            for (int j = 0; j < i; ++j) s -= M(i, j) * x[j * estride];
-            x[i * estride] = unit ? s : s / M(i, i);
-        }
-    } else {
-        for (int i = len - 1; i >= 0; --i) {
-            T s = alpha * x[i * estride];
-            for (int j = i + 1; j < len; ++j) s -= M(i, j) * x[j * estride];
-            x[i * estride] = unit ? s : s / M(i, i);
-        }
-    }
+    const int v0 = (int) blockIdx.x * TS_NV;
+    const int64_t es = left ? 1 : ldb, vs = left ? ldb : 1;  // strides of a vector's elements and between vectors
+    const bool mt = left ? trans != 0 : trans == 0;          // M(i, j) = A(j, i) when set
+    wg_trsm<T>(B + v0 * vs, es, vs, count - v0 < TS_NV ? count - v0 : TS_NV, len, A, lda, mt, (upper == 0) != mt,
+               unit != 0, alpha, reinterpret_cast<T *>(smem_raw));
 }
 
 // C's uplo triangle (diagonal included) <- alpha op(A) op(A)^T + beta C for op(A) n x k.
@@ -138,11 +125,17 @@ hipError_t launch_tile_potrf(hipStream_t s, int upper, T *A, int n, int64_t lda,
 template <typename T>
 hipError_t launch_tile_trsm(hipStream_t s, int left, int upper, int trans, int unit, int m, int n, T alpha,
                             const T *A, int64_t lda, T *B, int64_t ldb) {
-    const int count = left ? n : m;
-    if (count <= 0 || (left ? m : n) <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_trsm_vec<T>, dim3((count + NT - 1) / NT), dim3(NT), 0, s, m, n, alpha, A, lda, B, ldb, left,
-                       upper, trans, unit);
+    const int count = left ? n : m, len = left ? m : n;
+    if (count <= 0 || len <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_trsm_vec<T>, dim3((count + TS_NV - 1) / TS_NV), dim3(NT), (size_t) ts_lds_bytes<T>(len), s, m,
+                       n, alpha, A, lda, B, ldb, left, upper, trans, unit);
     return hipGetLastError();
+}
+
+template <typename T>
+hipError_t set_tileops_lds_limits() {
+    return hipFuncSetAttribute((const void *) k_trsm_vec<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int) ts_lds_bytes<T>(ts_len_lds<T>()));
 }
 
 template <typename T>
@@ -170,6 +163,7 @@ hipError_t launch_transpose(hipStream_t s, int m, int n, const T *src, int64_t l
 }
 
 #define HCAMD_TILEOPS_INSTANTIATE(T)                                                                             \
+    template hipError_t set_tileops_lds_limits<T>();                                                             \
     template hipError_t launch_tile_potrf<T>(hipStream_t, int, T *, int, int64_t, T *, int *);                   \
     template hipError_t launch_tile_trsm<T>(hipStream_t, int, int, int, int, int, int, T, const T *, int64_t, T *, \
                                             int64_t);                                                            \

@@ -12,6 +12,9 @@ namespace hcamd {
 // work: n * n elements of device scratch; info: first non-positive pivot (1-based) or 0.
 template <typename T>
 hipError_t launch_tile_potrf(hipStream_t s, int upper, T *A, int n, int64_t lda, T *work, int *info);
+// Once before the first launch_tile_trsm: lets its kernel use more than the default dynamic LDS.
+template <typename T>
+hipError_t set_tileops_lds_limits();
 // BLAS trsm on B (m x n, ld ldb): left ? op(A)^{-1} : (.) op(A)^{-1}, times alpha.
 template <typename T>
 hipError_t launch_tile_trsm(hipStream_t s, int left, int upper, int trans, int unit, int m, int n, T alpha,

@@ -167,3 +167,26 @@ def test_cholesky_flow_gemm_matches_oracle(ctx, dtype):
     # the other operand layouts are not part of that flow
     with pytest.raises(H.HCoreError, match="UNSUPPORTED"):
         H.HCore.gemm(1.0, A, B, 1.0, Ct, ctx, H.CompressionParameters(acc), opA="N", opB="N", cholesky=True)
+
+
+@pytest.mark.parametrize("dtype,tol", [(np.float64, 1e-13), (np.float32, 5e-5)])
+@pytest.mark.parametrize("order,r", [(1, 1), (31, 16), (32, 17), (33, 15), (97, 33), (286, 5), (500, 48), (700, 20),
+                                     (1200, 3)])
+def test_trsm_block_edges(ctx, order, r, dtype, tol):
+    """Solves whose order and vector count lie around the 32-row blocks, the 16 vectors of a workgroup
+    and the longest vectors held in LDS, all directions; the residual of a substitution is bounded by
+    order * eps * |op(A)| |x|, well inside the tolerances for these diagonally dominant matrices."""
+    H = _H()
+    rng = np.random.default_rng(order + r)
+    a = rng.standard_normal((order, order)) / order + 3.0 * np.eye(order)
+    for side, uplo, trans in (("L", "L", "N"), ("L", "L", "T"), ("L", "U", "N"), ("L", "U", "T"), ("R", "L", "T"),
+                              ("R", "U", "N")):
+        print(f"[case] trsm {order} {r} {side}{uplo}{trans} {dtype.__name__}", flush=True)
+        tri = np.tril(a) if uplo == "L" else np.triu(a)
+        rows, rank = (order, r) if side == "L" else (max(order, r), order)
+        v = rng.standard_normal((rows, rank))
+        B = H.CompressedTile.from_cholesky_factors(np.zeros((rows, rank)), v, max_rank=rank, dtype=dtype)
+        H.HCore.trsm(side, uplo, trans, "N", 0.5, H.DenseTile(tri, dtype=dtype), B, ctx)
+        op = tri.T if trans == "T" else tri
+        want = np.linalg.solve(op, 0.5 * v) if side == "L" else np.linalg.solve(op.T, 0.5 * v.T).T
+        assert rel_fro(B.cholesky_factors()[1], want) < tol
