@@ -253,14 +253,13 @@ hcorepp_status validate_tile(const hcorepp_tile *t, const char *name) {
     return HCOREPP_OK;
 }
 
-// Arena bytes of one plain recompression (workspace, rank word, sigma, Jacobi flags, QR panel scratch).
+// Arena bytes of one plain recompression (workspace, rank word, sigma, Jacobi flags, column norms).
 template <typename T>
 size_t recompress_arena_bytes(int64_t m, int64_t n, int64_t kmax, int64_t max_rank) {
     const WsLayout L = ws_layout<T>(m, n, kmax, max_rank);
     return aligned(sizeof(T) * L.total) + aligned(sizeof(int64_t) * 8) +
            aligned(sizeof(double) * (size_t) std::max<int64_t>(kmax, 1)) +
-           aligned(sizeof(int32_t) * JACOBI_MAX_SWEEPS) +
-           aligned(sizeof(T) * ((size_t) std::max(m, n) * 16 + 1024));
+           aligned(sizeof(int32_t) * JACOBI_MAX_SWEEPS) + aligned(sizeof(T) * JACOBI_ROWS_MAX);
 }
 
 template <typename T>
@@ -418,8 +417,7 @@ hcorepp_status recompress_plain(hcorepp_ctx *ctx, T alpha, const Holder<T> &ad, 
     if (ad.rows != m || bd.cols != n || bd.rows != arank)
         return fail(HCOREPP_ERR_INVALID, "operand shapes do not match C (%lldx%lld)", (long long) m,
                     (long long) n);
-    const int pb = pick_pb(std::max(m, n), kLdsBytes / (int64_t) sizeof(T));
-    if (pb == 0) return fail(HCOREPP_ERR_UNSUPPORTED, "tile too tall for the LDS panel (rows %lld)", (long long) m);
+    if (std::max(m, n) > 2048) return fail(HCOREPP_ERR_UNSUPPORTED, "tile too tall for the LDS panel (rows %lld)", (long long) m);
     if (std::min(m, K) > JACOBI_ROWS_MAX)
         return fail(HCOREPP_ERR_UNSUPPORTED, "stacked rank %lld exceeds the core SVD limit %d", (long long) K,
                     JACOBI_ROWS_MAX);
@@ -452,9 +450,8 @@ hcorepp_status recompress_plain(hcorepp_ctx *ctx, T alpha, const Holder<T> &ad, 
         for (int i = 0; i < 16; ++i) ctx->last_info[i] = info[i];
     }
     int32_t *jflags = (int32_t *) arena_take(ctx, sizeof(int32_t) * JACOBI_MAX_SWEEPS);
-    T *vpan = (T *) arena_take(ctx, sizeof(T) * ((size_t) std::max(m, n) * 16 + 1024));
-    HIP_TRY(launch_recomp_pre<T>(s, d, K, kLdsBytes, pb, jflags, ctx->pinned + HDR_WORDS,
-                                 vpan));
+    T *cn = (T *) arena_take(ctx, sizeof(T) * JACOBI_ROWS_MAX);
+    HIP_TRY(launch_recomp_pre<T>(s, d, K, jflags, ctx->pinned + HDR_WORDS, cn));
     // The plain form reads the new rank back with one stream synchronisation,
     // as the reference does (src/kernels/cuda/CudaKernels.cu:656-697).
     const int64_t *hdr = reinterpret_cast<const int64_t *>(d.ws + L.hdr);
@@ -467,7 +464,7 @@ hcorepp_status recompress_plain(hcorepp_ctx *ctx, T alpha, const Holder<T> &ad, 
     if (status & STATUS_NOCONV) return fail(HCOREPP_ERR_NUMERIC, "core Jacobi SVD did not converge");
     if (status & STATUS_TOO_BIG) return fail(HCOREPP_ERR_CAPACITY, "stacked rank exceeds the workspace");
     if (r < 1 || r > C->max_rank) return fail(HCOREPP_ERR_NUMERIC, "invalid rank %lld", (long long) r);
-    HIP_TRY(launch_recomp_post<T>(s, d, r, kLdsBytes, pb));
+    HIP_TRY(launch_recomp_post<T>(s, d, r));
     if (sigma_out && size_s > 0) {
         HIP_TRY(hipMemcpyAsync(sigma_out, d.sigma_out, sizeof(double) * size_s, hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));

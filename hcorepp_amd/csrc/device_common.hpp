@@ -56,6 +56,12 @@ __device__ __forceinline__ T wave_max(T v) {
     return v;
 }
 
+__device__ __forceinline__ int wave_sum_int(int v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
+    return v;
+}
+
 // Wave-wide sum (every lane gets the total); needs the whole wave active.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v);

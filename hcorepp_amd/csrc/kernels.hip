@@ -5,6 +5,9 @@
 #include "kernels.hpp"
 
 #include <cstring>
+#include <type_traits>
+
+#include "plain_qr.hpp"
 
 namespace hcamd {
 
@@ -29,16 +32,6 @@ __global__ void HCAMD_KERNEL k_stack(RecompDesc<T> d) {
     ph_stack<T>(d, blockIdx.x, gridDim.x);
 }
 
-template <typename T, int PB>
-__global__ void HCAMD_KERNEL k_qr(RecompDesc<T> d, int which) {
-    extern __shared__ unsigned char smem_raw[];
-    T *lds = reinterpret_cast<T *>(smem_raw);
-    Ws<T> w = ws_of(d);
-    const Dims z = dims_of(d, w);
-    if (which == 0) wg_geqrf<T, PB>(d.m, z.K, w.us, d.m, w.tau_u, w.t_u, lds);
-    else ph_qr_y<T, PB>(d, lds);
-}
-
 template <typename T>
 __global__ void HCAMD_KERNEL k_y(RecompDesc<T> d) {
     __shared__ T lds[GT_LDS_ELEMS];
@@ -46,156 +39,169 @@ __global__ void HCAMD_KERNEL k_y(RecompDesc<T> d) {
 }
 
 // ---------------------------------------------------------------------------
-// Multi-workgroup blocked QR of the plain form: one launch factors a panel (one workgroup,
-// window pivoting included for the QR of Y) and writes its unit-lower reflectors to `vpan`;
-// the next applies the block reflector to the trailing columns, a few column batches per
-// workgroup over the whole GPU.
+// Blocked QR of the plain form (plain_qr.hpp): one launch factors a panel (one workgroup, window pivoting
+// included for the QR of Y); the next applies its block reflector to the trailing columns, 16 columns
+// per workgroup over the whole GPU.  The operand's pointers and sizes come as arguments: the host knows
+// them, and a read of the workspace header at the start of every launch took 2 us.
 // ---------------------------------------------------------------------------
+
+// Set-up of the QR of Y: squared column norms (one wave per column), the identity permutation and J = 0.
 template <typename T>
-struct QrOperand {
-    T *A;
-    int m, ncols;
-    int64_t lda;
-    T *tau, *tsave;
-    bool pivot;
-};
-
-template <typename T, int PB>
-__device__ QrOperand<T> qr_operand(const RecompDesc<T> &d, const Ws<T> &w, const Dims &z, int which) {
-    if (which == 0) return QrOperand<T>{w.us, d.m, z.K, d.m, w.tau_u, w.t_u, false};
-    return QrOperand<T>{w.y, d.n, z.mu, d.n, w.tau_y, w.t_y, window_pivot_fits(d.n, z.mu, PB)};
-}
-
-// Squared norms of the columns of the QR operand `which` (all rows), one wave per column; the
-// window pivoting of the first panel reads them.
-template <typename T, int PB>
-__global__ void HCAMD_KERNEL k_qr_colnorms(RecompDesc<T> d, int which, T *cn) {
-    Ws<T> w = ws_of(d);
-    const Dims z = dims_of(d, w);
-    const QrOperand<T> q = qr_operand<T, PB>(d, w, z, which);
+__global__ void HCAMD_KERNEL k_qr_setup(PlainQr<T> q, int kk) {
     const int l = lane_id();
     for (int c = blockIdx.x * NWAVES + wave_id(); c < q.ncols; c += gridDim.x * NWAVES) {
-        const T *col = q.A + (int64_t) c * q.lda;
+        const T *col = q.A + (int64_t) c * q.m;
         T sum = T(0);
         for (int r = l; r < q.m; r += WAVE) sum += col[r] * col[r];
         sum = wave_sum(sum);
-        if (l == 0) cn[c] = sum;
+        if (l == 0) {
+            q.cn[c] = sum;
+            q.piv[c] = c;
+        }
     }
+    const int64_t tot = (int64_t) q.ncols * kk;
+    for (int64_t e = (int64_t) blockIdx.x * NT + threadIdx.x; e < tot; e += (int64_t) gridDim.x * NT) q.J[e] = T(0);
 }
 
-template <typename T, int PB>
-__global__ void HCAMD_KERNEL k_qr_panel(RecompDesc<T> d, int which, int j0, T *vpan, const T *cn) {
-    extern __shared__ unsigned char smem_raw[];
-    T *lds = reinterpret_cast<T *>(smem_raw);
-    Ws<T> w = ws_of(d);
-    const Dims z = dims_of(d, w);
-    const QrOperand<T> q = qr_operand<T, PB>(d, w, z, which);
-    if (which == 1 && j0 == 0) {
-        for (int c = threadIdx.x; c < q.ncols; c += NT) w.piv[c] = c;
-        __syncthreads();
-    }
-    if (which == 1 && q.pivot) {
-        // the QR of Y stops at the first panel whose trailing matrix is below the core-truncation
-        // level (as ph_qr_y); the launches after that return at once
-        if (w.hdr[HDR_KQ] > 0) return;
-        const int nsteps = q.m < q.ncols ? q.m : q.ncols;
-        const int jb = (nsteps - j0) < PB ? (nsteps - j0) : PB;
-        const T trail2 = window_pivot<T, PB>(q.m, q.ncols, q.A, q.lda, j0, jb, w.piv, lds, cn);
+template <typename T, int WAVES, int GROUPS>
+__global__ void __launch_bounds__(WAVES *WAVE) k_qr_panel(PlainQr<T> q, RecompDesc<T> d, int kk, int j0) {
+    __shared__ PanelLds<T, WAVES> lds;
+    // the QR of Y stops at the first panel whose trailing matrix is below the core-truncation
+    // level (as ph_qr_y); the launches after that return at once
+    if (q.pivot && q.hdr[HDR_KQ] > 0) return;
+    wg_panel<T, WAVES, GROUPS>(q, j0, lds, [&](T trail2) {
         if (j0 == 0) {
-            if (threadIdx.x == 0) w.hdr[HDR_STOP2] = __double_as_longlong((double) qr_y_stop2<T>(d, trail2, z.kk));
-        } else if (trail2 <= (T) __longlong_as_double(w.hdr[HDR_STOP2])) {
-            if (threadIdx.x == 0) {
-                w.hdr[HDR_KQ] = j0;
-                w.hdr[HDR_TRAIL2] = __double_as_longlong((double) trail2);
-            }
-            return;
+            if (threadIdx.x == 0) q.hdr[HDR_STOP2] = __double_as_longlong((double) qr_y_stop2<T>(d, trail2, kk));
+            return false;
         }
-        __syncthreads();
-        wg_geqrf_panel<T, PB>(q.m, q.ncols, q.A, q.lda, q.tau, q.tsave, lds, nullptr, w.hdr, j0);
-    } else {
-        wg_geqrf_panel<T, PB>(q.m, q.ncols, q.A, q.lda, q.tau, q.tsave, lds, q.pivot ? w.piv : nullptr, w.hdr, j0,
-                              q.pivot ? cn : nullptr);
-    }
+        if (!(trail2 <= (T) __longlong_as_double(q.hdr[HDR_STOP2]))) return false;
+        if (threadIdx.x == 0) {
+            q.hdr[HDR_KQ] = j0;
+            q.hdr[HDR_TRAIL2] = __double_as_longlong((double) trail2);
+        }
+        return true;
+    });
+}
+
+// Trailing update: workgroup x takes the columns at positions j0 + jb + 16 x .. + 15.  The block is read
+// once, kept in registers through both products and written back; pivoted, its rows of R go to J and the
+// squared norms below them to cn for the next panel's pivoting.
+template <typename T, int WAVES, int GROUPS>
+__global__ void __launch_bounds__(WAVES *WAVE) k_qr_update(PlainQr<T> q, int j0) {
+    __shared__ WyLds<T, WAVES> lds;
+    using MF = Mfma16<T>;
+    const int ln = lane_id(), i16 = ln & 15, k4 = ln >> 4, wv = wave_id();
     const int rows = q.m - j0;
-    wg_copy(vpan, lds, (int64_t) panel_ld(rows) * PB);
-}
-
-template <typename T, int PB, int RPT>
-__global__ void HCAMD_KERNEL k_qr_update(RecompDesc<T> d, int which, int j0, int cols_per_wg, const T *vpan,
-                                         T *cn) {
-    __shared__ T red[(NWAVES + 2) * WAVE];
-    Ws<T> w = ws_of(d);
-    const Dims z = dims_of(d, w);
-    const QrOperand<T> q = qr_operand<T, PB>(d, w, z, which);
-    if (which == 1 && w.hdr[HDR_KQ] > 0) return;  // the QR of Y stopped early
     const int nsteps = q.m < q.ncols ? q.m : q.ncols;
-    const int jb = (nsteps - j0) < PB ? (nsteps - j0) : PB;
-    const int c0 = j0 + jb + (int) blockIdx.x * cols_per_wg;
-    const int c1 = (c0 + cols_per_wg) < q.ncols ? (c0 + cols_per_wg) : q.ncols;
-    if (c0 >= c1) return;
-    apply_wy<T, PB, RPT>(vpan, panel_ld(q.m - j0), q.tsave + (int64_t) (j0 / PB) * PB * PB, q.m - j0, q.A + j0, q.lda,
-                         c0, c1, true, red);
+    const int jb = nsteps - j0 < PQ_NB ? nsteps - j0 : PQ_NB;
+    const int pos = j0 + jb + PQ_NB * (int) blockIdx.x + i16;
+    const bool cok = pos < q.ncols, wide = wide_columns(q.A, q.m);
+    auto column = [&](int p) { return q.pivot ? q.piv[p] : p; };
+    const int c = column(cok ? pos : j0);
+    const T *pcol = q.A + (int64_t) column(j0 + (i16 < jb ? i16 : 0)) * q.m + j0;
+    const T *prow[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const int k = MF::row(s, k4);
+        prow[s] = q.A + (int64_t) column(j0 + (k < jb ? k : 0)) * q.m + j0;
+    }
+    if (q.pivot && q.hdr[HDR_KQ] > 0) return;  // the QR of Y stopped early
+    T *col = q.A + (int64_t) c * q.m + j0;
+    T b[GROUPS][4];
+#pragma unroll
+    for (int t = 0; t < GROUPS; ++t) load_rows(col, 16 * (wv + WAVES * t) + 4 * k4, rows, cok, wide, b[t]);
+    const T *ts = q.tsave + (int64_t) (j0 / PQ_NB) * PQ_NB * PQ_NB;
+    const int pr = pq_prow<T>(i16);
+    // the panel's columns hold R on and above the diagonal: unit lower in the first group of rows
+    wy_block<T, WAVES, GROUPS>(
+            b,
+            [&](int t, T (&v)[4]) {
+                const int g = wv + WAVES * t;
+                load_rows(pcol, 16 * g + 4 * k4, rows, i16 < jb, wide, v);
+                if (g == 0) {
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        const int r = 4 * k4 + s;
+                        v[s] = r > i16 ? v[s] : T(r == i16 && i16 < jb);
+                    }
+                }
+            },
+            [&](int t, int s) {
+                const int r = 16 * (wv + WAVES * t) + pr, k = MF::row(s, k4);
+                if (k >= jb || r >= rows || r < k) return T(0);
+                return r == k ? T(1) : prow[s][r];
+            },
+            [&](int i, int j) { return i <= j ? ts[i + PQ_NB * j] : T(0); }, true, 0, lds);
+    T nsq = T(0);
+#pragma unroll
+    for (int t = 0; t < GROUPS; ++t) {
+        const int r = 16 * (wv + WAVES * t) + 4 * k4;
+        if (q.pivot) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                if (cok && r + s < jb) q.J[c + (int64_t) (j0 + r + s) * q.ncols] = b[t][s];
+                if (cok && r + s >= jb && r + s < rows) nsq = fma(b[t][s], b[t][s], nsq);
+            }
+        }
+        store_rows(col, r, rows, cok, wide, b[t]);
+    }
     if (q.pivot) {
-        // norms over rows [j0 + jb, m) of the updated columns, for the next panel's pivoting
+        nsq = col_sum(nsq);
+        if (k4 == 0) lds.part[wv][i16] = nsq;  // the partial products were read before the last barrier
         __syncthreads();
-        const int l = lane_id();
-        for (int c = c0 + wave_id(); c < c1; c += NWAVES) {
-            const T *col = q.A + (int64_t) c * q.lda;
+        if (threadIdx.x < PQ_NB && cok) {
             T sum = T(0);
-            for (int r = j0 + jb + l; r < q.m; r += WAVE) sum += col[r] * col[r];
-            sum = wave_sum(sum);
-            if (l == 0) cn[c] = sum;
+#pragma unroll
+            for (int ww = 0; ww < WAVES; ++ww) sum += lds.part[ww][i16];
+            q.cn[pos] = sum;
         }
     }
 }
 
-// Trailing update with the row-chunk count of the panel's rows (rows <= 512 for PB 16, <= 1024
-// for PB 8, <= 2048 for PB 4, as pick_pb guarantees).
-template <typename T, int PB>
-static void launch_qr_update(hipStream_t s, const RecompDesc<T> &d, int which, int j0, int rows, int grid, int cpw,
-                             const T *vpan, T *cn) {
-    const int chunks = (rows + WAVE * NWAVES - 1) / (WAVE * NWAVES);
-    if (chunks <= 1)
-        hipLaunchKernelGGL((k_qr_update<T, PB, 1>), dim3(grid), dim3(NT), 0, s, d, which, j0, cpw, vpan, cn);
-    else if (chunks <= 2)
-        hipLaunchKernelGGL((k_qr_update<T, PB, 2>), dim3(grid), dim3(NT), 0, s, d, which, j0, cpw, vpan, cn);
-    else if constexpr (PB <= 8) {
-        if (chunks <= 4)
-            hipLaunchKernelGGL((k_qr_update<T, PB, 4>), dim3(grid), dim3(NT), 0, s, d, which, j0, cpw, vpan, cn);
-        else if constexpr (PB <= 4)
-            hipLaunchKernelGGL((k_qr_update<T, PB, 8>), dim3(grid), dim3(NT), 0, s, d, which, j0, cpw, vpan, cn);
-    }
+// Waves and 16-row groups per wave for a block of `rows` rows (2048 at most).  Eight waves up to 1024 rows
+// (512 threads: 256 registers hold the 1024-row blocks, which 16 waves' 128 would spill).
+template <typename F>
+static void pq_shape(int rows, F f) {
+    const int g = (rows + 15) / 16;
+    if (g <= 8) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
+    else if (g <= 16) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 2>{});
+    else if (g <= 32) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
+    else if (g <= 64) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{});
+    else f(std::integral_constant<int, 16>{}, std::integral_constant<int, 8>{});
 }
 
-template <typename T, int PB>
-static hipError_t launch_qr_mw_pb(hipStream_t s, const RecompDesc<T> &d, int64_t lds_bytes, int which, int m,
-                                  int ncols, T *vpan) {
-    constexpr int NCB = WAVE / PB;
-    const int nsteps = m < ncols ? m : ncols;
-    T *cn = vpan + (int64_t) ((d.m > d.n ? d.m : d.n) + 1) * 16;  // after the largest panel (ld rows | 1)
-    if (which == 1)
-        hipLaunchKernelGGL((k_qr_colnorms<T, PB>), dim3((ncols + NWAVES - 1) / NWAVES), dim3(NT), 0, s, d, which, cn);
-    for (int j0 = 0; j0 < nsteps; j0 += PB) {
-        hipLaunchKernelGGL((k_qr_panel<T, PB>), dim3(1), dim3(NT), lds_bytes, s, d, which, j0, vpan, (const T *) cn);
-        const int jb = (nsteps - j0) < PB ? (nsteps - j0) : PB;
-        const int trail = ncols - (j0 + jb);
-        if (trail > 0) {
-            int cpw = NCB;
-            while ((trail + cpw - 1) / cpw > 512) cpw += NCB;
-            launch_qr_update<T, PB>(s, d, which, j0, m - j0, (trail + cpw - 1) / cpw, cpw, vpan, cn);
-        }
+template <typename T>
+static hipError_t launch_qr(hipStream_t s, const RecompDesc<T> &d, const PlainQr<T> &q, int kk) {
+    const int nsteps = q.m < q.ncols ? q.m : q.ncols;
+    if (q.pivot) {
+        const int grid = (q.ncols + NWAVES - 1) / NWAVES;
+        hipLaunchKernelGGL(k_qr_setup<T>, dim3(grid), dim3(NT), 0, s, q, kk);
+    }
+    for (int j0 = 0; j0 < nsteps; j0 += PQ_NB) {
+        const int jb = nsteps - j0 < PQ_NB ? nsteps - j0 : PQ_NB, trail = q.ncols - (j0 + jb);
+        pq_shape(q.m - j0, [&](auto waves, auto groups) {
+            constexpr int WV = decltype(waves)::value, GR = decltype(groups)::value;
+            hipLaunchKernelGGL((k_qr_panel<T, WV, GR>), dim3(1), dim3(WV * WAVE), 0, s, q, d, kk, j0);
+            if (trail > 0)
+                hipLaunchKernelGGL((k_qr_update<T, WV, GR>), dim3((trail + PQ_NB - 1) / PQ_NB), dim3(WV * WAVE), 0, s, q,
+                                   j0);
+        });
     }
     return hipGetLastError();
 }
 
 template <typename T>
-static hipError_t launch_qr_mw(hipStream_t s, const RecompDesc<T> &d, int64_t lds_bytes, int pb, int which, int m,
-                               int ncols, T *vpan) {
-    switch (pb) {
-        case 16: return launch_qr_mw_pb<T, 16>(s, d, lds_bytes, which, m, ncols, vpan);
-        case 8: return launch_qr_mw_pb<T, 8>(s, d, lds_bytes, which, m, ncols, vpan);
-        default: return launch_qr_mw_pb<T, 4>(s, d, lds_bytes, which, m, ncols, vpan);
-    }
+__global__ void HCAMD_KERNEL k_fill_identity(T *I, int64_t n) {
+    for (int64_t e = (int64_t) blockIdx.x * NT + threadIdx.x; e < n * n; e += (int64_t) gridDim.x * NT)
+        I[e] = ((e % n) == (e / n)) ? T(1) : T(0);
+}
+
+template <typename T>
+hipError_t launch_fill_identity(hipStream_t s, T *I, int64_t n) {
+    int64_t grid = (n * n + NT - 1) / NT;
+    if (grid > 1024) grid = 1024;
+    hipLaunchKernelGGL(k_fill_identity<T>, dim3((unsigned) (grid > 0 ? grid : 1)), dim3(NT), 0, s, I, n);
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -208,16 +214,34 @@ static hipError_t launch_qr_mw(hipStream_t s, const RecompDesc<T> &d, int64_t ld
 constexpr int JW_THREADS = 512;                  // the one-workgroup Jacobi
 constexpr int64_t JW_LDS_BYTES = 150 * 1024;     // its LDS: the workgroup has the CU to itself
 
+// Squared norms of the core's columns (the rows of R_Y), one wave per column.
 template <typename T>
-__global__ void HCAMD_KERNEL k_core(RecompDesc<T> d, int32_t *flags) {
-    __shared__ T gbuf[CORE_LDS_ELEMS];
-    ph_core<T>(d, gbuf);
+__global__ void HCAMD_KERNEL k_core_norms(const T *J, int mu, int kk, T *rn) {
+    for (int j = blockIdx.x * NWAVES + wave_id(); j < kk; j += gridDim.x * NWAVES) {
+        T sum = T(0);
+        for (int r = lane_id(); r < mu; r += WAVE) {
+            const T v = J[r + (int64_t) j * mu];
+            sum += v * v;
+        }
+        sum = wave_sum(sum);
+        if (lane_id() == 0) rn[j] = sum;
+    }
+}
+
+// Core width from those norms (ph_core_width), ||J||_F^2, and the Jacobi's flags.
+template <typename T>
+__global__ void HCAMD_KERNEL k_core_size(RecompDesc<T> d, const T *norms, int32_t *flags) {
+    __shared__ T rn[CORE_LDS_ELEMS];
+    Ws<T> w = ws_of(d);
+    const Dims z = dims_of(d, w);
+    for (int j = threadIdx.x; j < z.kk; j += NT) rn[j] = norms[j];
     for (int i = threadIdx.x; i < JACOBI_MAX_SWEEPS; i += NT) flags[i] = 0;
+    __syncthreads();
+    ph_core_width<T>(d, rn);
     if (threadIdx.x == 0) {
-        Ws<T> w = ws_of(d);
-        const Dims z = dims_of(d, w);
-        // gbuf[j] = ||R_Y[j:, :]||_F^2 after ph_core_size, so ||J||_F^2 = gbuf[0] - gbuf[kt]
-        const T fro2 = z.kk > 0 ? gbuf[0] - (z.kt < z.kk ? gbuf[z.kt] : T(0)) : T(0);
+        // rn[j] = ||R_Y[j:, :]||_F^2 now, so ||J||_F^2 = rn[0] - rn[kt]
+        const int kt = (int) w.hdr[HDR_KT];
+        const T fro2 = z.kk > 0 ? rn[0] - (kt < z.kk ? rn[kt] : T(0)) : T(0);
         w.hdr[HDR_JFRO2] = __double_as_longlong((double) fro2);
     }
 }
@@ -240,6 +264,8 @@ __global__ void __launch_bounds__(JW_THREADS) k_jacobi_wg(RecompDesc<T> d) {
     T *Jl = lds + gram_jacobi_lds<T>(NW), *Vl = Jl + (int64_t) ldj * nc;
     const bool jin = (int64_t) ldj * nc <= cap, vin = (int64_t) (ldj + ldv) * nc <= cap;
     int sweeps;
+    if (!vin)
+        for (ColWalk p(threadIdx.x, JW_THREADS, nc); p.c < nc; p.next()) w.v1[p.i + (int64_t) p.c * nc] = T(p.i == p.c);
     if (nc < 1) {
         sweeps = 0;
     } else if (jin) {
@@ -260,6 +286,7 @@ __global__ void __launch_bounds__(JW_THREADS) k_jacobi_wg(RecompDesc<T> d) {
             for (ColWalk p(threadIdx.x, JW_THREADS, nc); p.c < nc; p.next())
                 w.v1[p.i + (int64_t) p.c * nc] = Vl[p.i + p.c * ldv];
     } else {
+        __syncthreads();
         sweeps = wg_gram_jacobi<T>(w.j, rows, rows, nc, w.v1, nc, nc, fro2, stop, JACOBI_MAX_SWEEPS, NW, lds);
     }
     if (threadIdx.x == 0) w.hdr[HDR_SWEEPS] = sweeps;
@@ -320,17 +347,55 @@ static void launch_jacobi_step(hipStream_t s, const MwJacobi<T> &m, int sweep, i
 }
 static_assert(JACOBI_ROWS_MAX <= 16 * MW_WAVES * 6, "the widest k_jacobi_step holds the tallest core");
 
-// `launched` sweeps of the multi-workgroup Jacobi, or -1 after the one-workgroup one.
+// Singular values (column norms of the orthogonalised core), one wave per column.
 template <typename T>
-__global__ void HCAMD_KERNEL k_svd_finish(RecompDesc<T> d, const int32_t *flags, int launched) {
+__global__ void HCAMD_KERNEL k_svd_sigma(RecompDesc<T> d) {
     Ws<T> w = ws_of(d);
+    const Dims z = dims_of(d, w);
+    const int j = blockIdx.x * NWAVES + wave_id();
+    if (j >= z.kt) return;
+    const T *zj = w.j + (int64_t) j * z.mu;
+    T s = T(0);
+    for (int r = lane_id(); r < z.mu; r += WAVE) s += zj[r] * zj[r];
+    s = wave_sum(s);
+    if (lane_id() == 0) w.sig[j] = sqrt(s);
+}
+
+// Their descending order, four threads per column, and (workgroup 0) the rank rule.  `launched` sweeps of
+// the multi-workgroup Jacobi, or -1 after the one-workgroup one.
+template <typename T>
+__global__ void HCAMD_KERNEL k_svd_rank(RecompDesc<T> d, const int32_t *flags, int launched) {
+    __shared__ T sig[JACOBI_ROWS_MAX];
+    Ws<T> w = ws_of(d);
+    const Dims z = dims_of(d, w);
+    const int kt = z.kt;
+    for (int j = threadIdx.x; j < kt; j += NT) sig[j] = w.sig[j];
+    __syncthreads();
+    const int j = (int) blockIdx.x * (NT / 4) + (int) threadIdx.x / 4, part = threadIdx.x % 4;
+    int pos = 0;
+    if (j < kt) {
+        const T sj = order_key(sig[j]);
+        for (int k = part; k < kt; k += 4) {
+            const T sk = order_key(sig[k]);
+            pos += (sk > sj) || (sk == sj && k < j);
+        }
+    }
+    pos += __shfl_xor(pos, 1, WAVE);
+    pos += __shfl_xor(pos, 2, WAVE);
+    if (j < kt && part == 0) {
+        w.perm[pos] = j;
+        if (d.sigma_out) d.sigma_out[pos] = (double) sig[j];
+    }
+    if (blockIdx.x != 0) return;
+    if (d.sigma_out)
+        for (int i = kt + threadIdx.x; i < z.kk; i += NT) d.sigma_out[i] = 0.0;
     int sweeps = launched < 0 ? (int) w.hdr[HDR_SWEEPS] : launched;
     for (int s = 0; s < launched; ++s)
         if (flags[s] == 0) {
             sweeps = s;
             break;
         }
-    ph_svd_finish<T>(d, sweeps);
+    ph_rank<T>(d, sig, sweeps);
 }
 
 // The whole core SVD.  Cores that may be wide (kk columns are known here) have their width read back
@@ -339,8 +404,16 @@ __global__ void HCAMD_KERNEL k_svd_finish(RecompDesc<T> d, const int32_t *flags,
 // The sweeps are launched in chunks; the host reads the last sweep's flag between chunks.
 template <typename T>
 static hipError_t launch_core_svd(hipStream_t s, const RecompDesc<T> &d, int mu, int kk, int32_t *flags,
-                                  volatile int64_t *host) {
-    hipLaunchKernelGGL(k_core<T>, dim3(1), dim3(NT), 0, s, d, flags);
+                                  volatile int64_t *host, T *scratch) {
+    const WsLayout L = ws_layout<T>(d.m, d.n, d.kmax, d.max_rank);
+    auto finish = [&](int kt, int launched) {
+        hipLaunchKernelGGL(k_svd_sigma<T>, dim3((kt + NWAVES - 1) / NWAVES), dim3(NT), 0, s, d);
+        hipLaunchKernelGGL(k_svd_rank<T>, dim3((kt + NT / 4 - 1) / (NT / 4)), dim3(NT), 0, s, d, flags, launched);
+        return hipGetLastError();
+    };
+    hipLaunchKernelGGL(k_core_norms<T>, dim3((kk + NWAVES - 1) / NWAVES), dim3(NT), 0, s, (const T *) (d.ws + L.j), mu,
+                       kk, scratch);
+    hipLaunchKernelGGL(k_core_size<T>, dim3(1), dim3(NT), 0, s, d, (const T *) scratch, flags);
     hipError_t e;
     int kt = kk;
     T fro2 = T(0);
@@ -358,12 +431,12 @@ static hipError_t launch_core_svd(hipStream_t s, const RecompDesc<T> &d, int mu,
     }
     if (kt < MW_MIN_COLS) {
         hipLaunchKernelGGL(k_jacobi_wg<T>, dim3(1), dim3(JW_THREADS), JW_LDS_BYTES, s, d);
-        hipLaunchKernelGGL(k_svd_finish<T>, dim3(1), dim3(NT), 0, s, d, flags, -1);
-        return hipGetLastError();
+        return finish(kt, -1);
     }
-    const WsLayout L = ws_layout<T>(d.m, d.n, d.kmax, d.max_rank);
     const int nblk = (kt + GJ_B - 1) / GJ_B, nbp = nblk + (nblk & 1);
     const MwJacobi<T> m{d.ws + L.j, d.ws + L.v1, d.ws + L.j2, flags, mu, kt, nbp, fro2};
+    e = launch_fill_identity<T>(s, m.v, kt);
+    if (e != hipSuccess) return e;
     // most cores converge within 5 to 8 sweeps: the first five are launched at once, then one at a time
     int launched = 0, chunk = 5;
     while (launched < JACOBI_MAX_SWEEPS) {
@@ -380,24 +453,87 @@ static hipError_t launch_core_svd(hipStream_t s, const RecompDesc<T> &d, int mu,
         chunk = 1;
     }
     launch_jacobi_step<T>(s, m, launched, 0, 1);
-    hipLaunchKernelGGL(k_svd_finish<T>, dim3(1), dim3(NT), 0, s, d, flags, launched);
-    return hipGetLastError();
+    return finish(kt, launched);
 }
 
-template <typename T, int PB>
-__global__ void HCAMD_KERNEL k_recon(RecompDesc<T> d, int cols_per_wg) {
-    extern __shared__ unsigned char smem_raw[];
-    const int c0 = blockIdx.x * cols_per_wg;
-    ph_recon<T, PB>(d, blockIdx.y, c0, c0 + cols_per_wg, reinterpret_cast<T *>(smem_raw));
-}
-
-template <typename T>
-__global__ void HCAMD_KERNEL k_finish(RecompDesc<T> d) {
-    ph_finish<T>(d, blockIdx.x, gridDim.x);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        Ws<T> w = ws_of(d);
-        *d.crank = w.hdr[HDR_RANK];
+// Reconstruction of the plain form, 16 columns of the new rank per workgroup, side blockIdx.y:
+//   0: C_U[:, c] = Q_U [z_perm(c) / sigma; 0]  (z: column of J = P R_Y^T after the Jacobi; P, the pivoting of
+//      the QR of Y, is applied when J is built)
+//   1: C_V[c, :] = (Q_Y [v1_perm(c) sigma; 0])^T
+// The block stays in registers from its first to its last reflector panel and goes straight to the tile
+// (C_V transposed: 16 consecutive elements per store).
+template <typename T, int WAVES, int GROUPS>
+__global__ void __launch_bounds__(WAVES *WAVE) k_recon(RecompDesc<T> d) {
+    __shared__ WyLds<T, WAVES> lds;
+    __shared__ int32_t cols[PQ_MAX_COLS];  // the columns that hold the reflectors
+    using MF = Mfma16<T>;
+    Ws<T> w = ws_of(d);
+    const Dims z = dims_of(d, w);
+    const int r = (int) w.hdr[HDR_RANK], side = (int) blockIdx.y;
+    const int ln = lane_id(), i16 = ln & 15, k4 = ln >> 4, wv = wave_id();
+    const int c = PQ_NB * (int) blockIdx.x + i16;
+    const bool cok = c < r && c < z.kt;
+    const int rows = side ? d.n : d.m, filled = side ? z.kt : z.mu;
+    const T *src = side ? w.v1 : w.j;
+    const int j = cok ? w.perm[c] : 0;
+    const T sg = cok ? w.sig[j] : T(0);
+    T b[GROUPS][4];
+#pragma unroll
+    for (int t = 0; t < GROUPS; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int row = 16 * (wv + WAVES * t) + 4 * k4 + s;
+            const T v = (cok && row < filled) ? src[row + (int64_t) j * filled] : T(0);
+            b[t][s] = side ? v * sg : (sg > T(0) ? v / sg : T(0));
+        }
+    const T *A = side ? w.y : w.us, *tsave = side ? w.t_y : w.t_u;  // ld rows
+    // [v1 sigma; 0] vanishes below row kt, where reflectors kt.. of Q_Y act as the identity (each is zero
+    // above its own row), so only the first kt are applied
+    const int nref = side ? (z.kt < z.kk ? z.kt : z.kk) : z.mu;
+    const int pr = pq_prow<T>(i16);
+    const bool wide = wide_columns(A, rows);
+    for (int i = threadIdx.x; i < nref; i += WAVES * WAVE) cols[i] = side ? w.piv[i] : i;
+    __syncthreads();
+    for (int p = (nref + PQ_NB - 1) / PQ_NB - 1; p >= 0; --p) {
+        const int j0 = p * PQ_NB, jb = nref - j0 < PQ_NB ? nref - j0 : PQ_NB;
+        const T *ts = tsave + (int64_t) p * PQ_NB * PQ_NB;
+        const T *pcol = A + (int64_t) cols[j0 + (i16 < jb ? i16 : 0)] * rows;
+        const T *prow[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) prow[s] = A + (int64_t) cols[j0 + (MF::row(s, k4) < jb ? MF::row(s, k4) : 0)] * rows;
+        // the panel is unit lower from row j0 on (a multiple of 16: one mixed group)
+        wy_block<T, WAVES, GROUPS>(
+                b,
+                [&](int t, T (&v)[4]) {
+                    const int g = wv + WAVES * t;
+                    load_rows(pcol, 16 * g + 4 * k4, rows, i16 < jb && g >= p, wide, v);
+                    if (g == p) {
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) {
+                            const int rr = 4 * k4 + s;
+                            v[s] = rr > i16 ? v[s] : T(rr == i16 && i16 < jb);
+                        }
+                    }
+                },
+                [&](int t, int s) {
+                    const int row = 16 * (wv + WAVES * t) + pr, k = MF::row(s, k4);
+                    if (k >= jb || row >= rows || row < j0 + k) return T(0);
+                    return row == j0 + k ? T(1) : prow[s][row];
+                },
+                [&](int i, int jj) { return (i <= jj && jj < jb) ? ts[i + PQ_NB * jj] : T(0); }, false, p, lds);
     }
+    if (c >= r) return;
+    T *cu = d.cdata, *cv = d.cdata + (int64_t) d.m * d.max_rank;
+#pragma unroll
+    for (int t = 0; t < GROUPS; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int row = 16 * (wv + WAVES * t) + 4 * k4 + s;
+            if (row < rows) {
+                if (side) cv[c + (int64_t) row * r] = b[t][s];
+                else cu[row + (int64_t) c * d.m] = b[t][s];
+            }
+        }
 }
 
 __global__ void k_set_i64(int64_t *p, int64_t v) {
@@ -417,20 +553,6 @@ __global__ void HCAMD_KERNEL k_readjust_ddc(const T *W, int64_t m, int64_t n, T 
             cdata[e] = ((f % n) == (f / n)) ? T(1) : T(0);
         }
     }
-}
-
-template <typename T>
-__global__ void HCAMD_KERNEL k_fill_identity(T *I, int64_t n) {
-    for (int64_t e = (int64_t) blockIdx.x * NT + threadIdx.x; e < n * n; e += (int64_t) gridDim.x * NT)
-        I[e] = ((e % n) == (e / n)) ? T(1) : T(0);
-}
-
-template <typename T>
-hipError_t launch_fill_identity(hipStream_t s, T *I, int64_t n) {
-    int64_t grid = (n * n + NT - 1) / NT;
-    if (grid > 1024) grid = 1024;
-    hipLaunchKernelGGL(k_fill_identity<T>, dim3((unsigned) (grid > 0 ? grid : 1)), dim3(NT), 0, s, I, n);
-    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -524,7 +646,7 @@ __global__ void HCAMD_KERNEL k_batched(const BatchEntry<T> *entries, const int32
             __syncthreads();
             ph_core_size<T>(d, lds);
             ph_learned_size<T>(d, lds);
-            ph_core_build<T, false>(d);
+            ph_core_build<T>(d);
             ph_core_qr<T, PB>(d, lds);
             t_qry = HCAMD_TSTAMP();
             ph_svd_nov<T>(d);
@@ -602,29 +724,6 @@ bool pb_fits(int64_t rows, int pb, int64_t lds_elems) {
     return qr_lds_elems(rows, pb) <= lds_elems;
 }
 
-template <typename T, int PB>
-static hipError_t launch_qr_pb(hipStream_t s, const RecompDesc<T> &d, int64_t lds_bytes, int which) {
-    hipLaunchKernelGGL((k_qr<T, PB>), dim3(1), dim3(NT), lds_bytes, s, d, which);
-    return hipGetLastError();
-}
-
-template <typename T, int PB>
-static hipError_t launch_recon_pb(hipStream_t s, const RecompDesc<T> &d, int64_t lds_bytes, int r) {
-    const int cols = 64 / PB;  // one column batch of the compact-WY application per workgroup
-    const int nch = (r + cols - 1) / cols;
-    hipLaunchKernelGGL((k_recon<T, PB>), dim3(nch > 0 ? nch : 1, 2), dim3(NT), lds_bytes, s, d, cols);
-    return hipGetLastError();
-}
-
-template <typename T>
-static hipError_t launch_qr(hipStream_t s, const RecompDesc<T> &d, int64_t lds_bytes, int pb, int which) {
-    switch (pb) {
-        case 16: return launch_qr_pb<T, 16>(s, d, lds_bytes, which);
-        case 8: return launch_qr_pb<T, 8>(s, d, lds_bytes, which);
-        default: return launch_qr_pb<T, 4>(s, d, lds_bytes, which);
-    }
-}
-
 static int clamp_grid(int64_t work) {
     int64_t g = (work + NT - 1) / NT;
     if (g > 1024) g = 1024;
@@ -633,33 +732,32 @@ static int clamp_grid(int64_t work) {
 }
 
 template <typename T>
-hipError_t launch_recomp_pre(hipStream_t s, const RecompDesc<T> &d, int64_t K, int64_t lds_bytes, int pb,
-                             int32_t *jflags, int64_t *host, T *vpan) {
+hipError_t launch_recomp_pre(hipStream_t s, const RecompDesc<T> &d, int64_t K, int32_t *jflags, int64_t *host,
+                             T *cn) {
     const int64_t m = d.m, n = d.n;
     const int64_t mu = m < K ? m : K;
     const int64_t kk = n < mu ? n : mu;
     hipLaunchKernelGGL(k_stack<T>, dim3(clamp_grid(m * K)), dim3(NT), 0, s, d);
-    hipError_t e = (K >= MW_MIN_QR_COLS) ? launch_qr_mw<T>(s, d, lds_bytes, pb, 0, (int) m, (int) K, vpan)
-                                                 : launch_qr<T>(s, d, lds_bytes, pb, 0);
+    const WsLayout L = ws_layout<T>(m, n, d.kmax, d.max_rank);
+    int64_t *hdr = reinterpret_cast<int64_t *>(d.ws + L.hdr);
+    const PlainQr<T> qu{d.ws + L.us, d.ws + L.tau_u, d.ws + L.t_u, nullptr, nullptr, nullptr, hdr, (int) m, (int) K, 0};
+    const PlainQr<T> qy{d.ws + L.y, d.ws + L.tau_y, d.ws + L.t_y, d.ws + L.j, cn,
+                        reinterpret_cast<int32_t *>(d.ws + L.piv), hdr, (int) n, (int) mu, 1};
+    hipError_t e = launch_qr<T>(s, d, qu, (int) kk);
     if (e != hipSuccess) return e;
     const int ytiles = (int) (((n + GT_M - 1) / GT_M) * ((mu + GT_N - 1) / GT_N));
     hipLaunchKernelGGL(k_y<T>, dim3(ytiles), dim3(NT), 0, s, d);
-    e = (mu >= MW_MIN_QR_COLS) ? launch_qr_mw<T>(s, d, lds_bytes, pb, 1, (int) n, (int) mu, vpan)
-                                       : launch_qr<T>(s, d, lds_bytes, pb, 1);
+    e = launch_qr<T>(s, d, qy, (int) kk);
     if (e != hipSuccess) return e;
-    return launch_core_svd<T>(s, d, (int) mu, (int) kk, jflags, host);
+    return launch_core_svd<T>(s, d, (int) mu, (int) kk, jflags, host, cn);
 }
 
 template <typename T>
-hipError_t launch_recomp_post(hipStream_t s, const RecompDesc<T> &d, int64_t r, int64_t lds_bytes, int pb) {
-    hipError_t e;
-    switch (pb) {
-        case 16: e = launch_recon_pb<T, 16>(s, d, lds_bytes, (int) r); break;
-        case 8: e = launch_recon_pb<T, 8>(s, d, lds_bytes, (int) r); break;
-        default: e = launch_recon_pb<T, 4>(s, d, lds_bytes, (int) r); break;
-    }
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_finish<T>, dim3(clamp_grid(r * d.n)), dim3(NT), 0, s, d);
+hipError_t launch_recomp_post(hipStream_t s, const RecompDesc<T> &d, int64_t r) {
+    pq_shape(d.m > d.n ? d.m : d.n, [&](auto waves, auto groups) {
+        constexpr int WV = decltype(waves)::value, GR = decltype(groups)::value;
+        hipLaunchKernelGGL((k_recon<T, WV, GR>), dim3((unsigned) ((r + PQ_NB - 1) / PQ_NB), 2), dim3(WV * WAVE), 0, s, d);
+    });
     return hipGetLastError();
 }
 
@@ -706,9 +804,6 @@ template <typename T>
 hipError_t set_kernel_lds_limits(int64_t lds_bytes) {
     // Allow the dynamic-LDS kernels to use more than the default 64 KB.
     const void *fns[] = {
-            (const void *) k_qr<T, 16>, (const void *) k_qr<T, 8>, (const void *) k_qr<T, 4>,
-            (const void *) k_qr_panel<T, 16>, (const void *) k_qr_panel<T, 8>, (const void *) k_qr_panel<T, 4>,
-            (const void *) k_recon<T, 16>, (const void *) k_recon<T, 8>, (const void *) k_recon<T, 4>,
             (const void *) k_batched<T, 16>, (const void *) k_batched<T, 8>, (const void *) k_batched<T, 4>,
     };
     for (const void *f : fns) {
@@ -722,9 +817,9 @@ hipError_t set_kernel_lds_limits(int64_t lds_bytes) {
 #define HCAMD_INSTANTIATE(T)                                                                                     \
     template hipError_t launch_gemm<T>(hipStream_t, int, int, int, T, const T *, int64_t, bool, const T *,      \
                                        int64_t, bool, T, T *, int64_t);                                          \
-    template hipError_t launch_recomp_pre<T>(hipStream_t, const RecompDesc<T> &, int64_t, int64_t, int, int32_t *, \
-                                             int64_t *, T *);                                                    \
-    template hipError_t launch_recomp_post<T>(hipStream_t, const RecompDesc<T> &, int64_t, int64_t, int);        \
+    template hipError_t launch_recomp_pre<T>(hipStream_t, const RecompDesc<T> &, int64_t, int32_t *, int64_t *,  \
+                                             T *);                                                               \
+    template hipError_t launch_recomp_post<T>(hipStream_t, const RecompDesc<T> &, int64_t);                      \
     template hipError_t launch_readjust_ddc<T>(hipStream_t, const T *, int64_t, int64_t, T *);                   \
     template hipError_t launch_fill_identity<T>(hipStream_t, T *, int64_t);                                      \
     template hipError_t launch_batched<T>(hipStream_t, const BatchEntry<T> *, const int32_t *, int64_t,          \

@@ -60,19 +60,16 @@ template <typename T>
 hipError_t launch_gemm(hipStream_t s, int M, int N, int Kd, T alpha, const T *A, int64_t lda, bool ta, const T *B,
                        int64_t ldb, bool tb, T beta, T *C, int64_t ldc);
 // Cores of at least MW_MIN_COLS columns run their Jacobi over many workgroups (that path
-// synchronises the stream, for the core's width and between sweep chunks); QRs of at least
-// MW_MIN_QR_COLS columns run panel by panel with multi-workgroup trailing updates.  `jflags`:
-// JACOBI_MAX_SWEEPS device ints; `host`: one pinned word; `vpan`: max(m, n) * 16 + 1024 elements of
-// device scratch (the panel, then column norms).
+// synchronises the stream, for the core's width and between sweep chunks).  `jflags`:
+// JACOBI_MAX_SWEEPS device ints; `host`: two pinned words; `cn`: min(m, K) elements of device scratch
+// (column norms).  m, n <= 2048.
 // The records of the multi-workgroup Jacobi (at most 32 elements per column and 1 K) fit the workspace
 // region they use, (kk + 17) kk elements, from 48 columns on.
 constexpr int MW_MIN_COLS = 112;
-constexpr int MW_MIN_QR_COLS = 128;
 template <typename T>
-hipError_t launch_recomp_pre(hipStream_t s, const RecompDesc<T> &d, int64_t K, int64_t lds_bytes, int pb,
-                             int32_t *jflags, int64_t *host, T *vpan);
+hipError_t launch_recomp_pre(hipStream_t s, const RecompDesc<T> &d, int64_t K, int32_t *jflags, int64_t *host, T *cn);
 template <typename T>
-hipError_t launch_recomp_post(hipStream_t s, const RecompDesc<T> &d, int64_t r, int64_t lds_bytes, int pb);
+hipError_t launch_recomp_post(hipStream_t s, const RecompDesc<T> &d, int64_t r);
 hipError_t launch_set_i64(hipStream_t s, int64_t *p, int64_t v);
 template <typename T>
 hipError_t launch_readjust_ddc(hipStream_t s, const T *W, int64_t m, int64_t n, T *cdata);

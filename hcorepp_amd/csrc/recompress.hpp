@@ -1079,15 +1079,66 @@ __device__ void ph_y(const RecompDesc<T> &d, int wg, int nwg, T *lds) {
 // of that level, and never below a requested fixed rank.
 // ph_core_size writes kt to the header and leaves in lds: rn[j] = ||R_Y[j:, :]||_F^2 (kk values)
 // followed by a lower bound of the rank threshold; ph_core_build then builds
-// J = P R_Y[0:kt, :]^T (mu x kt, ld mu; P the pivoting of the QR of Y) and V1 = I (kt x kt).  `lds` holds >= kk + NWAVES values.
+// J = P R_Y[0:kt, :]^T (mu x kt, ld mu; P the pivoting of the QR of Y).  `lds` holds >= kk + NWAVES values.
+// The width from the squared row norms rn[0..kk) (rows the QR of Y did not form count as what it left):
+// rn becomes the suffix sums and rn[kk] the threshold bound.  Wave 0 scans 64 rows at a time from the end (one
+// thread's loops over 600 rows took 100 us).
+template <typename T>
+__device__ void ph_core_width(const RecompDesc<T> &d, T *rn) {
+    Ws<T> w = ws_of(d);
+    const Dims z = dims_of(d, w);
+    const int kk = z.kk, l = lane_id();
+    const int kq = (w.hdr[HDR_KQ] > 0 && w.hdr[HDR_KQ] < kk) ? (int) w.hdr[HDR_KQ] : kk;
+    const T trail2 = kq < kk ? (T) __longlong_as_double(w.hdr[HDR_TRAIL2]) : T(0);
+    if (wave_id() == 0) {
+        T carry = trail2;
+        for (int j0 = (kq - 1) / WAVE * WAVE; j0 >= 0; j0 -= WAVE) {
+            T v = j0 + l < kq ? rn[j0 + l] : T(0);
+#pragma unroll
+            for (int off = 1; off < WAVE; off <<= 1) {
+                const T o = __shfl_down(v, off, WAVE);
+                if (l + off < WAVE) v += o;
+            }
+            v += carry;
+            if (j0 + l < kq) rn[j0 + l] = v;  // ||R_Y[j:, :]||_F^2
+            carry = read_lane(v, 0);
+        }
+        for (int j = kq + l; j < kk; j += WAVE) rn[j] = trail2;
+        wave_fence();
+        const T fro2 = kk > 0 ? rn[0] : T(0);
+        const T delta = Eps<T>::value * sqrt(fro2);
+        int kt = kk;
+        // threshold the rank rule will use, bounded below (sigma_0 >= ||J||_F / sqrt(kk))
+        const T thr_lo = d.truncated_svd ? T(d.accuracy) * sqrt(fro2 / T(kk > 0 ? kk : 1)) : T(d.accuracy);
+        if (thr_lo > T(64) * delta) {
+            for (int j0 = 0; j0 < kk && kt == kk; j0 += WAVE) {
+                const int j = j0 + l;
+                const unsigned long long below = __ballot(j >= 1 && j < kk && sqrt(rn[j < kk ? j : 0]) <= delta);
+                if (below) kt = j0 + __ffsll(below) - 1;
+            }
+        }
+        if (d.fixed_rank > 0) {
+            const int fr = d.fixed_rank < kk ? d.fixed_rank : kk;
+            if (kt < fr) kt = fr;
+        }
+        if (kt > kq) kt = kq;  // only kq rows of R_Y exist (the rest were left below the stop test)
+        if (kt < 1) kt = kk < 1 ? 0 : 1;
+        if (l == 0) {
+            w.hdr[HDR_KT] = kt;
+            w.hdr[HDR_CQR] = 0;
+            rn[kk] = thr_lo;
+        }
+    }
+    __syncthreads();
+}
+
 template <typename T>
 __device__ void ph_core_size(const RecompDesc<T> &d, T *lds) {
     Ws<T> w = ws_of(d);
     const Dims z = dims_of(d, w);
     const int mu = z.mu, kk = z.kk, n = d.n, l = lane_id();
-    // rows of R_Y the QR of Y computed (all kk unless it stopped early) and the norm it left
+    // rows of R_Y the QR of Y computed (all kk unless it stopped early)
     const int kq = (w.hdr[HDR_KQ] > 0 && w.hdr[HDR_KQ] < kk) ? (int) w.hdr[HDR_KQ] : kk;
-    const T trail2 = kq < kk ? (T) __longlong_as_double(w.hdr[HDR_TRAIL2]) : T(0);
     T *rn = lds;  // suffix sums, then the threshold bound at rn[kk]
     for (int j = wave_id(); j < kq; j += NWAVES) {
         T sum = T(0);
@@ -1099,42 +1150,10 @@ __device__ void ph_core_size(const RecompDesc<T> &d, T *lds) {
         if (l == 0) rn[j] = sum;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int j = kq; j < kk; ++j) rn[j] = trail2;  // rows never formed: bounded by what was left
-        T acc = trail2;
-        for (int j = kq - 1; j >= 0; --j) {
-            acc += rn[j];
-            rn[j] = acc;  // ||R_Y[j:, :]||_F^2
-        }
-        const T fro2 = kk > 0 ? rn[0] : T(0);
-        const T delta = Eps<T>::value * sqrt(fro2);
-        int kt = kk;
-        // threshold the rank rule will use, bounded below (sigma_0 >= ||J||_F / sqrt(kk))
-        const T thr_lo = d.truncated_svd ? T(d.accuracy) * sqrt(fro2 / T(kk > 0 ? kk : 1)) : T(d.accuracy);
-        if (thr_lo > T(64) * delta) {
-            for (int j = 1; j < kk; ++j) {
-                if (sqrt(rn[j]) <= delta) {
-                    kt = j;
-                    break;
-                }
-            }
-        }
-        if (d.fixed_rank > 0) {
-            const int fr = d.fixed_rank < kk ? d.fixed_rank : kk;
-            if (kt < fr) kt = fr;
-        }
-        if (kt > kq) kt = kq;  // only kq rows of R_Y exist (the rest were left below the stop test)
-        if (kt < 1) kt = kk < 1 ? 0 : 1;
-        w.hdr[HDR_KT] = kt;
-        w.hdr[HDR_CQR] = 0;
-        rn[kk] = thr_lo;
-    }
-    __syncthreads();
+    ph_core_width<T>(d, rn);
 }
 
-// WITH_V: also set V1 = I for the Jacobi that accumulates the right rotations (the batched
-// form's Jacobi keeps no V and skips it).
-template <typename T, bool WITH_V = true>
+template <typename T>
 __device__ void ph_core_build(const RecompDesc<T> &d) {
     Ws<T> w = ws_of(d);
     const Dims z = dims_of(d, w);
@@ -1144,16 +1163,7 @@ __device__ void ph_core_build(const RecompDesc<T> &d) {
     if (mu > 0)
         for (ColWalk p(threadIdx.x, NT, mu); p.c < kt; p.next())
             w.j[w.piv[p.i] + (int64_t) p.c * mu] = (p.i >= p.c) ? w.y[p.c + (int64_t) p.i * n] : T(0);
-    if (WITH_V && kt > 0)
-        for (ColWalk p(threadIdx.x, NT, kt); p.c < kt; p.next())
-            w.v1[p.i + (int64_t) p.c * kt] = (p.i == p.c) ? T(1) : T(0);
     __syncthreads();
-}
-
-template <typename T>
-__device__ void ph_core(const RecompDesc<T> &d, T *lds) {
-    ph_core_size<T>(d, lds);
-    ph_core_build<T>(d);
 }
 
 // Second QR of a tall core (batched form): J (mu x kt) = Q2 R2, after which the Jacobi runs on the
@@ -1183,41 +1193,38 @@ constexpr int JACOBI_ROWS_MAX = 768;
 // LDS of the core set-up: ph_core_size's row norms and threshold.
 constexpr int CORE_LDS_ELEMS = JACOBI_ROWS_MAX + NWAVES + 8;
 
-// Tail of the core SVD once the Jacobi has converged (`sweeps` used): singular values, their
-// descending order, the rank rule and the header words.
+// The rank rule and the header words, by one workgroup, from the kt singular values sig (any order; those
+// beyond the truncated core width kt are below eps * ||J||_F: zero): the first index i >= 1 in descending order
+// whose value is below the threshold, i.e. the number of values not below it, at least 1.
 template <typename T>
-__device__ void ph_svd_finish(const RecompDesc<T> &d, int sweeps) {
+__device__ void ph_rank(const RecompDesc<T> &d, const T *sig, int sweeps) {
     Ws<T> w = ws_of(d);
     const Dims z = dims_of(d, w);
-    const int mu = z.mu, kk = z.kk, kt = z.kt, K = z.K;
-    __shared__ int s_nan;
-    if (threadIdx.x == 0) s_nan = 0;
+    const int kk = z.kk, kt = z.kt, K = z.K;
+    __shared__ int s_nan, s_above;
+    __shared__ T s_max[NWAVES];
+    if (threadIdx.x == 0) s_nan = s_above = 0;
     __syncthreads();
-    const int l = lane_id();
-    // the orthogonalised core: J (mu rows) or, after the core QR, R2 (kt rows)
-    const bool cqr = w.hdr[HDR_CQR] != 0;
-    const T *zc = cqr ? w.j2 : w.j;
-    const int zrows = cqr ? kt : mu;
-    for (int j = wave_id(); j < kt; j += NWAVES) {
-        const T *zj = zc + (int64_t) j * zrows;
-        T s = 0;
-        for (int r = l; r < zrows; r += WAVE) s += zj[r] * zj[r];
-        s = wave_sum(s);
-        if (l == 0) {
-            w.sig[j] = sqrt(s);
-            if (!(s == s) || s > T(1e300)) atomicOr(&s_nan, 1);
-        }
-    }
-    __syncthreads();
+    T top = T(-INFINITY);
+    int nan = 0;
     for (int j = threadIdx.x; j < kt; j += NT) {
-        const T sj = order_key(w.sig[j]);
-        int pos = 0;
-        for (int k = 0; k < kt; ++k) {
-            const T sk = order_key(w.sig[k]);
-            pos += (sk > sj) || (sk == sj && k < j);
-        }
-        w.perm[pos] = j;
+        const T s = sig[j];
+        nan |= !(s == s) || s * s > T(1e300);
+        top = order_key(s) > top ? order_key(s) : top;
     }
+    top = wave_max(top);
+    if (lane_id() == 0) s_max[wave_id()] = top;
+    if (__ballot(nan) && lane_id() == 0) atomicOr(&s_nan, 1);
+    __syncthreads();
+    T s0 = s_max[0];
+#pragma unroll
+    for (int i = 1; i < NWAVES; ++i) s0 = s_max[i] > s0 ? s_max[i] : s0;
+    if (kt < 1) s0 = T(0);
+    const T thr = d.truncated_svd ? T(d.accuracy) * s0 : T(d.accuracy);
+    int above = 0;
+    for (int j = threadIdx.x; j < kt; j += NT) above += !(order_key(sig[j]) < thr);
+    above = wave_sum_int(above);
+    if (lane_id() == 0) atomicAdd(&s_above, above);
     __syncthreads();
     if (threadIdx.x == 0) {
         const int size_s = kk;
@@ -1227,17 +1234,7 @@ __device__ void ph_svd_finish(const RecompDesc<T> &d, int sweeps) {
             if (rk > K) rk = K;
             if (rk > size_s) rk = size_s;
         } else {
-            // singular values beyond the truncated core width kt are below eps * ||J||_F: zero
-            rk = size_s;
-            const T s0 = kt > 0 ? w.sig[w.perm[0]] : T(0);
-            const T thr = d.truncated_svd ? T(d.accuracy) * s0 : T(d.accuracy);
-            for (int i = 1; i < size_s; ++i) {
-                const T si = i < kt ? w.sig[w.perm[i]] : T(0);
-                if (si < thr) {
-                    rk = i;
-                    break;
-                }
-            }
+            rk = s_above + (T(0) < thr ? 0 : size_s - kt);
         }
         if (rk < 1) rk = 1;
         if (rk > d.max_rank) rk = d.max_rank;
@@ -1250,11 +1247,43 @@ __device__ void ph_svd_finish(const RecompDesc<T> &d, int sweeps) {
         if (sweeps >= JACOBI_MAX_SWEEPS) st |= STATUS_NOCONV;
         if (s_nan) st |= STATUS_NAN;
         w.hdr[HDR_STATUS] |= st;
-        if (d.sigma_out) {
-            for (int i = 0; i < size_s; ++i) d.sigma_out[i] = i < kt ? (double) w.sig[w.perm[i]] : 0.0;
-        }
     }
     __syncthreads();
+}
+
+// Tail of the core SVD once the Jacobi has converged (`sweeps` used): singular values, their
+// descending order, the rank rule and the header words.
+template <typename T>
+__device__ void ph_svd_finish(const RecompDesc<T> &d, int sweeps) {
+    Ws<T> w = ws_of(d);
+    const Dims z = dims_of(d, w);
+    const int mu = z.mu, kk = z.kk, kt = z.kt;
+    const int l = lane_id();
+    // the orthogonalised core: J (mu rows) or, after the core QR, R2 (kt rows)
+    const bool cqr = w.hdr[HDR_CQR] != 0;
+    const T *zc = cqr ? w.j2 : w.j;
+    const int zrows = cqr ? kt : mu;
+    for (int j = wave_id(); j < kt; j += NWAVES) {
+        const T *zj = zc + (int64_t) j * zrows;
+        T s = 0;
+        for (int r = l; r < zrows; r += WAVE) s += zj[r] * zj[r];
+        s = wave_sum(s);
+        if (l == 0) w.sig[j] = sqrt(s);
+    }
+    __syncthreads();
+    for (int j = threadIdx.x; j < kt; j += NT) {
+        const T sj = order_key(w.sig[j]);
+        int pos = 0;
+        for (int k = 0; k < kt; ++k) {
+            const T sk = order_key(w.sig[k]);
+            pos += (sk > sj) || (sk == sj && k < j);
+        }
+        w.perm[pos] = j;
+    }
+    __syncthreads();
+    if (d.sigma_out)
+        for (int i = threadIdx.x; i < kk; i += NT) d.sigma_out[i] = i < kt ? (double) w.sig[w.perm[i]] : 0.0;
+    ph_rank<T>(d, w.sig, sweeps);
 }
 
 // ---------------------------------------------------------------------------
@@ -1407,76 +1436,6 @@ __device__ void ph_recon_nov(const RecompDesc<T> &d, T *lds) {
     // [X^T U; 0] vanishes below row kt, where reflectors kt.. of Q_Y act as the identity
     wg_apply_q<T, PB>(n, kt < kk ? kt : kk, w.y, n, w.t_y, w.vtmp, n, 0, r, lds);
     HCAMD_SUB_END(t_aq, w.hdr, 4);
-}
-
-// ---------------------------------------------------------------------------
-// Phase: reconstruction of columns [c0, c1) of the new rank.
-//   side 0: C_U[:, c] = Q_U [z_perm(c) / sigma; 0]  (z: column of J = P R_Y^T after the Jacobi, or
-//           of Q2 R2 W after the core QR; P, the pivoting of the QR of Y, is applied when J is built)
-//   side 1: vtmp[:, c] = Q_Y [v1_perm(c) * sigma; 0]
-// ---------------------------------------------------------------------------
-template <typename T, int PB>
-__device__ void ph_recon(const RecompDesc<T> &d, int side, int c0, int c1, T *lds) {
-    Ws<T> w = ws_of(d);
-    const Dims z = dims_of(d, w);
-    const int r = (int) w.hdr[HDR_RANK];
-    if (c1 > r) c1 = r;
-    if (c0 >= c1) return;
-    const int m = d.m, n = d.n, mu = z.mu, kk = z.kk, kt = z.kt;
-    if (side == 0 && w.hdr[HDR_CQR]) {
-        T *B = d.cdata;  // ld m
-        // left factor of the core J = Q2 R2: Q2 [Z2 / sigma; 0] in rows [0, mu), zero below
-        for (ColWalk p(threadIdx.x, NT, m); p.c < c1 - c0; p.next()) {
-            const int i = p.i, c = c0 + p.c;
-            T v = T(0);
-            if (i < kt && c < kt) {
-                const int j = w.perm[c];
-                const T sg = w.sig[j];
-                v = (sg > T(0)) ? w.j2[i + (int64_t) j * kt] / sg : T(0);
-            }
-            B[i + (int64_t) c * m] = v;
-        }
-        __syncthreads();
-        wg_apply_q<T, PB>(mu, kt, w.j, mu, w.t_j, B, m, c0, c1, lds);
-        __syncthreads();
-        HCAMD_SUB_BEGIN(t_aq);
-        wg_apply_q<T, PB>(m, mu, w.us, m, w.t_u, B, m, c0, c1, lds);
-        HCAMD_SUB_END(t_aq, w.hdr, 4);
-    } else if (side == 0) {
-        T *B = d.cdata;  // ld m
-        // the core's left factor Z / sigma in rows [0, mu) (J's rows are in Q_U's basis order)
-        for (ColWalk p(threadIdx.x, NT, m); p.c < c1 - c0; p.next()) {
-            const int i = p.i, c = c0 + p.c;
-            T v = T(0);
-            if (i < mu && c < kt) {
-                const int j = w.perm[c];
-                const T sg = w.sig[j];
-                v = (sg > T(0)) ? w.j[i + (int64_t) j * mu] / sg : T(0);
-            }
-            B[i + (int64_t) c * m] = v;
-        }
-        __syncthreads();
-        HCAMD_SUB_BEGIN(t_aq);
-        wg_apply_q<T, PB>(m, mu, w.us, m, w.t_u, B, m, c0, c1, lds);
-        HCAMD_SUB_END(t_aq, w.hdr, 4);
-    } else {
-        T *B = w.vtmp;  // ld n
-        for (ColWalk p(threadIdx.x, NT, n); p.c < c1 - c0; p.next()) {
-            const int i = p.i, c = c0 + p.c;
-            T v = T(0);
-            if (i < kt && c < kt) {
-                const int j = w.perm[c];
-                v = w.v1[i + (int64_t) j * kt] * w.sig[j];
-            }
-            B[i + (int64_t) c * n] = v;
-        }
-        __syncthreads();
-        // [v1 sigma; 0] vanishes below row kt, where reflectors kt.. of Q_Y act as the identity
-        // (each is zero above its own row), so only the first kt are applied
-        HCAMD_SUB_BEGIN(t_aq);
-        wg_apply_q<T, PB>(n, kt < kk ? kt : kk, w.y, n, w.t_y, B, n, c0, c1, lds);
-        HCAMD_SUB_END(t_aq, w.hdr, 4);
-    }
 }
 
 // Phase: C_V (r x n, ld r) = vtmp^T.
