@@ -201,6 +201,75 @@ __device__ void wg_gemm(int M, int N, int Kd, T alpha, const T *A, int64_t lda, 
 }
 
 // ---------------------------------------------------------------------------
+// Products too small to fill the GPU with 64 x 64 tiles: one workgroup of 8 waves per 32 x 32 tile, the
+// waves splitting K (16 at a time) and each holding the whole tile as 2 x 2 matrix-core blocks.  The operands
+// go from memory to registers in the matrix cores' layout, four 16-deep chunks in flight per wave, without
+// LDS or barriers until the waves' sums are added up at the end, so a K of 512 is one memory round trip.
+// (The 64 x 64 form walks K in 16 staged chunks in one workgroup, 38 us for a 64 x 72 product of K = 512; the
+// three products of C += (U V)(U V) with a dense 512 x 512 C took 62 us, 27 here.)  fa(i, k), fb(k, j) and epi(i, j, v) as in wg_gemm_tile_core; k_lo: the operands vanish before it.
+// ---------------------------------------------------------------------------
+constexpr int GS_T = 32, GS_WAVES = 8, GS_CH = 4;
+constexpr int GS_LDS_ELEMS = GS_WAVES * 16 * (GS_T + 1);
+template <typename T, typename FA, typename FB, typename EPI>
+__device__ __forceinline__ void wg_gemm_small(int M, int N, int Kd, const FA &fa, const FB &fb, const EPI &epi, int ti,
+                                              int tj, T *lds, int k_lo = 0) {
+    using MF = Mfma16<T>;
+    const int l = lane_id(), i16 = l & 15, k4 = l >> 4, w = wave_id();
+    const int i0 = ti * GS_T, j0 = tj * GS_T;
+    typename MF::acc acc[2][2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[p][q] = MF::zero();
+    k_lo &= ~15;
+    for (int k0 = k_lo + 16 * w; k0 < Kd; k0 += 16 * GS_WAVES * GS_CH) {
+        T a[GS_CH][2][4], b[GS_CH][2][4];
+#pragma unroll
+        for (int c = 0; c < GS_CH; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    // a chunk's 16 terms may be summed in any order: lane k4 takes k0 + 4 k4 .. + 3
+                    const int k = k0 + 16 * GS_WAVES * c + 4 * k4 + s, i = i0 + 16 * h + i16, j = j0 + 16 * h + i16;
+                    a[c][h][s] = (k < Kd && i < M) ? fa(i, k) : T(0);
+                    b[c][h][s] = (k < Kd && j < N) ? fb(k, j) : T(0);
+                }
+#pragma unroll
+        for (int c = 0; c < GS_CH; ++c) {
+            if (k0 + 16 * GS_WAVES * c >= Kd) break;
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) acc[p][q] = MF::mma(a[c][p][s], b[c][q][s], acc[p][q]);
+        }
+    }
+    // the waves' sums, 16 rows of the tile at a time
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        if (p) __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) lds[(w * 16 + MF::row(v, k4)) * (GS_T + 1) + 16 * q + i16] = acc[p][q][v];
+        __syncthreads();
+        const int i = threadIdx.x % 16, j = threadIdx.x / 16;  // 512 threads: one element each
+        T sum = T(0);
+#pragma unroll
+        for (int ww = 0; ww < GS_WAVES; ++ww) sum += lds[(ww * 16 + i) * (GS_T + 1) + j];
+        const int gi = i0 + 16 * p + i, gj = j0 + j;
+        if (gi < M && gj < N) epi(gi, gj, sum);
+    }
+}
+
+// Whether a product of M x N output takes that form: fewer than 256 tiles of 64 x 64, one per CU.
+__host__ __device__ inline bool gemm_is_small(int64_t M, int64_t N) {
+    return ((M + GT_M - 1) / GT_M) * ((N + GT_N - 1) / GT_N) < 256;
+}
+
+// ---------------------------------------------------------------------------
 // Mixed-precision tile GEMM: C = op(A) op(B) (alpha = 1, beta = 0) for FP64 operands with the
 // products formed on the FP32 matrix cores (v_mfma_f32_16x16x4f32) with FP32 accumulation, made
 // exact by an error-free split of the operands (the Ozaki scheme).  Each row i of op(A) is scaled

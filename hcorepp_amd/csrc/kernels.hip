@@ -28,6 +28,20 @@ __global__ void HCAMD_KERNEL k_gemm(int M, int N, int Kd, T alpha, const T *A, i
 }
 
 template <typename T>
+__global__ void __launch_bounds__(GS_WAVES *WAVE) k_gemm_small(int M, int N, int Kd, T alpha, const T *A, int64_t lda,
+                                                              int ta, const T *B, int64_t ldb, int tb, T beta, T *C,
+                                                              int64_t ldc) {
+    __shared__ T lds[GS_LDS_ELEMS];
+    auto fa = [=](int i, int k) -> T { return ta ? A[k + (int64_t) i * lda] : A[i + (int64_t) k * lda]; };
+    auto fb = [=](int k, int j) -> T { return tb ? B[j + (int64_t) k * ldb] : B[k + (int64_t) j * ldb]; };
+    auto epi = [=](int gi, int gj, T v) {
+        T *c = C + gi + (int64_t) gj * ldc;
+        *c = (beta == T(0)) ? alpha * v : alpha * v + beta * *c;
+    };
+    wg_gemm_small<T>(M, N, Kd, fa, fb, epi, blockIdx.x, blockIdx.y, lds);
+}
+
+template <typename T>
 __global__ void HCAMD_KERNEL k_stack(RecompDesc<T> d) {
     ph_stack<T>(d, blockIdx.x, gridDim.x);
 }
@@ -36,6 +50,20 @@ template <typename T>
 __global__ void HCAMD_KERNEL k_y(RecompDesc<T> d) {
     __shared__ T lds[GT_LDS_ELEMS];
     ph_y<T>(d, blockIdx.x, gridDim.x, lds);
+}
+
+// The same by 32 x 32 tiles (wg_gemm_small), for a Y of fewer than 256 tiles of 64 x 64.
+template <typename T>
+__global__ void __launch_bounds__(GS_WAVES *WAVE) k_y_small(RecompDesc<T> d, int K, int mu) {
+    __shared__ T lds[GS_LDS_ELEMS];
+    const WsLayout L = ws_layout<T>(d.m, d.n, d.kmax, d.max_rank);
+    const StackedV<T> fa = stacked_v(d, K);
+    const T *us = d.ws + L.us;
+    T *y = d.ws + L.y;
+    const int64_t ldu = d.m, ldy = d.n;
+    auto fb = [=](int k, int j) -> T { return k < j ? T(0) : us[j + (int64_t) k * ldu]; };  // R_U^T
+    auto epi = [=](int gi, int gj, T v) { y[gi + (int64_t) gj * ldy] = v; };
+    wg_gemm_small<T>(d.n, mu, K, fa, fb, epi, blockIdx.x, blockIdx.y, lds, (int) blockIdx.y * GS_T);
 }
 
 // ---------------------------------------------------------------------------
@@ -702,6 +730,12 @@ template <typename T>
 hipError_t launch_gemm(hipStream_t s, int M, int N, int Kd, T alpha, const T *A, int64_t lda, bool ta, const T *B,
                        int64_t ldb, bool tb, T beta, T *C, int64_t ldc) {
     if (M <= 0 || N <= 0) return hipSuccess;
+    if (gemm_is_small(M, N)) {
+        dim3 grid((M + GS_T - 1) / GS_T, (N + GS_T - 1) / GS_T);
+        hipLaunchKernelGGL(k_gemm_small<T>, grid, dim3(GS_WAVES * WAVE), 0, s, M, N, Kd, alpha, A, lda, (int) ta, B, ldb,
+                           (int) tb, beta, C, ldc);
+        return hipGetLastError();
+    }
     dim3 grid((M + GT_M - 1) / GT_M, (N + GT_N - 1) / GT_N);
     hipLaunchKernelGGL(k_gemm<T>, grid, dim3(NT), 0, s, M, N, Kd, alpha, A, lda, (int) ta, B, ldb, (int) tb, beta,
                        C, ldc);
@@ -746,7 +780,11 @@ hipError_t launch_recomp_pre(hipStream_t s, const RecompDesc<T> &d, int64_t K, i
     hipError_t e = launch_qr<T>(s, d, qu, (int) kk);
     if (e != hipSuccess) return e;
     const int ytiles = (int) (((n + GT_M - 1) / GT_M) * ((mu + GT_N - 1) / GT_N));
-    hipLaunchKernelGGL(k_y<T>, dim3(ytiles), dim3(NT), 0, s, d);
+    if (gemm_is_small(n, mu))
+        hipLaunchKernelGGL(k_y_small<T>, dim3((unsigned) ((n + GS_T - 1) / GS_T), (unsigned) ((mu + GS_T - 1) / GS_T)),
+                           dim3(GS_WAVES * WAVE), 0, s, d, (int) K, (int) mu);
+    else
+        hipLaunchKernelGGL(k_y<T>, dim3(ytiles), dim3(NT), 0, s, d);
     e = launch_qr<T>(s, d, qy, (int) kk);
     if (e != hipSuccess) return e;
     return launch_core_svd<T>(s, d, (int) mu, (int) kk, jflags, host, cn);
