@@ -1326,6 +1326,7 @@ hcorepp_status hcorepp_syrk_batch_d(hcorepp_ctx *ctx, int64_t n, const hcorepp_t
     if (!ctx || n < 0 || (n > 0 && (!A || !C))) return fail(HCOREPP_ERR_INVALID, "bad arguments");
     std::vector<CholSyrk> jobs;
     size_t scratch = 0;
+    int64_t max_n = 0, max_rank = 0;
     for (int64_t i = 0; i < n; ++i) {
         if ((st = validate_tile<double>(&A[i], "A[i]")) || (st = validate_tile<double>(&C[i], "C[i]"))) return st;
         if (A[i].type != HCOREPP_COMPRESSED || C[i].type != HCOREPP_DENSE || C[i].rows != C[i].cols ||
@@ -1334,6 +1335,8 @@ hcorepp_status hcorepp_syrk_batch_d(hcorepp_ctx *ctx, int64_t n, const hcorepp_t
                         (long long) i, (long long) i);
         scratch += aligned(sizeof(double) * (size_t) (A[i].rank * A[i].rank)) +
                    aligned(sizeof(double) * (size_t) (A[i].rows * A[i].rank));
+        max_n = std::max(max_n, A[i].rows);
+        max_rank = std::max(max_rank, A[i].rank);
     }
     if ((st = arena_begin(ctx, scratch + sizeof(CholSyrk) * (size_t) (n + 1) + 4096))) return st;
     for (int64_t i = 0; i < n; ++i) {
@@ -1345,7 +1348,7 @@ hcorepp_status hcorepp_syrk_batch_d(hcorepp_ctx *ctx, int64_t n, const hcorepp_t
     }
     CholSyrk *dj;
     if ((st = upload_jobs(ctx, jobs, &dj))) return st;
-    HIP_TRY(launch_syrk(ctx->stream, dj, (int) jobs.size()));
+    HIP_TRY(launch_syrk(ctx->stream, dj, (int) jobs.size(), (int) max_n, (int) max_rank));
     return HCOREPP_OK;
 }
 

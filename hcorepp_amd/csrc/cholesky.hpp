@@ -31,7 +31,8 @@ hipError_t launch_potrf(hipStream_t s, T *A, int n, int64_t lda, int *info);
 hipError_t launch_trsm_v(hipStream_t s, const CholTrsm *jobs, int n, int max_rank, int len);
 // Once before the first launch_trsm_v: lets its kernel use more than the default dynamic LDS.
 hipError_t set_cholesky_lds_limits();
-hipError_t launch_syrk(hipStream_t s, const CholSyrk *jobs, int n);
+// n jobs of up to max_n rows and ranks up to max_rank.
+hipError_t launch_syrk(hipStream_t s, const CholSyrk *jobs, int n, int max_n, int max_rank);
 hipError_t launch_transpose_factors(hipStream_t s, const CholTrans *jobs, int n);
 
 }  // namespace hcamd

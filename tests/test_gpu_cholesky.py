@@ -170,3 +170,44 @@ def test_tlr_cholesky_batched_mixed_backward_error(ctx):
     A = M.dense_block_range(0, M.n)
     be = np.linalg.norm(A - Ld @ Ld.T) / np.linalg.norm(A)
     assert be < 5e-6, be
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 65, 96, 97, 129])
+def test_potrf_syrk_block_edges(ctx, n):
+    """Sizes at the edges of the 32-column blocks and 32 x 32 tiles, leading dimensions beyond n, ranks around a tile's
+    width.  potrf: |S - L L^T| <= (n + 1) eps |L| |L|^T elementwise (each element of L takes at most n products and
+    one division or root), with a factor 4 for the quotients' and roots' last bit; syrk: three products of n, r
+    and r terms and a subtraction."""
+    H, HC, OC = _mods()
+    import ctypes as C
+    eps = np.finfo(np.float64).eps
+    rng = np.random.default_rng(n)
+
+    def padded(a, extra):
+        t = H.DenseTile(np.vstack([a, np.full((extra, n), 7.0)]))
+        t.rows = n
+        return t
+
+    G = rng.standard_normal((n, n))
+    S = G @ G.T + np.eye(n)
+    D = padded(S, n % 3)
+    H._check(H.lib().hcorepp_potrf_d(ctx.h, C.byref(D.c())))
+    ctx.sync()
+    L = D.to_numpy()
+    assert np.array_equal(np.triu(L, 1), np.zeros((n, n)))
+    aL = np.abs(L)
+    assert np.all(np.abs(S - L @ L.T) <= 4 * (n + 1) * eps * (aL @ aL.T + np.abs(S)))
+    ranks = sorted({r for r in (0, 1, 31, 32, 33, 65) if r <= n})
+    us = [rng.standard_normal((n, r)) for r in ranks]
+    vs = [rng.standard_normal((r, n)) for r in ranks]
+    Bs = [H.CompressedTile(u, v, max_rank=max(ranks) + 1) for u, v in zip(us, vs)]
+    Cs = [padded(G, 2) for _ in ranks]
+    H._check(H.lib().hcorepp_syrk_batch_d(ctx.h, len(Bs), (H._Tile * len(Bs))(*[b.c() for b in Bs]),
+                                          (H._Tile * len(Cs))(*[c.c() for c in Cs])))
+    ctx.sync()
+    for r, u, v, c in zip(ranks, us, vs, Cs):
+        out = c.to_numpy()
+        assert np.array_equal(np.triu(out, 1), np.zeros((n, n)))
+        au, av = np.abs(u), np.abs(v)
+        bound = 2 * (n + 2 * r + 3) * eps * (au @ (av @ av.T) @ au.T + np.abs(G))
+        assert np.all(np.abs(np.tril(out - (G - u @ (v @ v.T) @ u.T))) <= bound), r
