@@ -14,7 +14,7 @@ error on a sample, ranks on all updates):
   fp64_exact    exact core (truncated only at the rounding level of its QR)
   fp64_learned  core presized by the trained BF16 rank MLP, exact acceptance test
   fp64_rule     the same tolerance applied directly to the pivoted R factor
-  mixed_rule    factor products on FP32 matrix cores (FP32 accumulation over error-free slices
+  mixed_rule    factor products on FP16 matrix cores (FP32 accumulation over error-free slices
                 of the FP64 operands), core truncated by the same tolerance rule as fp64_rule
   mixed_learned the same products with the learned core sizing of fp64_learned
 The headline `value` is the fastest form whose error stays <= 1e-8.  Also
@@ -645,7 +645,7 @@ def main():
                         f"the dropped part <= {LEARNED_TOL} * accuracy, else exact core), persistent kernel",
         "fp64_rule": f"batched FP64, core truncated where the pivoted R factor's dropped part <= {LEARNED_TOL} * "
                      f"accuracy, persistent kernel",
-        "mixed_rule": "batched, factor products on FP32 matrix cores with FP32 accumulation over error-free slices "
+        "mixed_rule": "batched, factor products on FP16 matrix cores with FP32 accumulation over error-free slices "
                       f"of the FP64 operands, QR/SVD/truncation FP64, core truncated as fp64_rule (tol {LEARNED_TOL}), "
                       "persistent kernel",
         "mixed_learned": "batched, mixed-precision factor products as mixed_rule, core presized by the BF16 rank MLP "

@@ -206,7 +206,8 @@ __device__ void wg_gemm(int M, int N, int Kd, T alpha, const T *A, int64_t lda, 
 // go from memory to registers in the matrix cores' layout, four 16-deep chunks in flight per wave, without
 // LDS or barriers until the waves' sums are added up at the end, so a K of 512 is one memory round trip.
 // (The 64 x 64 form walks K in 16 staged chunks in one workgroup, 38 us for a 64 x 72 product of K = 512; the
-// three products of C += (U V)(U V) with a dense 512 x 512 C took 62 us, 27 here.)  fa(i, k), fb(k, j) and epi(i, j, v) as in wg_gemm_tile_core; k_lo: the operands vanish before it.
+// three products of C += (U V)(U V) with a dense 512 x 512 C took 62 us, 27 here.)  fa(i, k), fb(k, j) and
+// epi(i, j, v) as in wg_gemm_tile_core; k_lo: the operands vanish before it.
 // ---------------------------------------------------------------------------
 constexpr int GS_T = 32, GS_WAVES = 8, GS_CH = 4;
 constexpr int GS_LDS_ELEMS = GS_WAVES * 16 * (GS_T + 1);
@@ -271,71 +272,122 @@ __host__ __device__ inline bool gemm_is_small(int64_t M, int64_t N) {
 
 // ---------------------------------------------------------------------------
 // Mixed-precision tile GEMM: C = op(A) op(B) (alpha = 1, beta = 0) for FP64 operands with the
-// products formed on the FP32 matrix cores (v_mfma_f32_16x16x4f32) with FP32 accumulation, made
+// products formed on the FP16 matrix cores (v_mfma_f32_16x16x16_f16) with FP32 accumulation, made
 // exact by an error-free split of the operands (the Ozaki scheme).  Each row i of op(A) is scaled
 // by a power of two 2^ea_i above its largest magnitude and cut into MS_SLICES slices: integers
 // x_s of at most MS_BITS bits with op(A)[i, k] = 2^ea_i sum_s x_s 2^(-MS_BITS (s+1)) + (a rest
-// below 2^(ea_i - MS_BITS MS_SLICES - 1)); each column of op(B) likewise.  A slice product summed
-// over one 16-deep K chunk is an integer of magnitude at most 16 * 2^(2 MS_BITS) = 2^24, exact
-// in FP32 whatever order the matrix core sums in; every slice pair (s, t) with s + t < MS_SLICES
-// is summed per chunk in FP32 and added to the FP64 result with its power-of-two weight.  The
-// error is the dropped slices: about 2^-40 of 2^(ea_i + eb_j) per term (FP64 rounding for the
+// below 2^(ea_i - MS_BITS MS_SLICES - 1)); each column of op(B) likewise.  FP16 holds every such integer
+// exactly (|x_0| <= 2^10, the later ones 2^9).  The products of the slice pairs with s + t = d are summed in FP32
+// over one 16-deep K chunk: for d = 0 and 1, which carry the result's leading bits, at most 2^24 and exact
+// in whatever order the matrix core sums; d = 2 and 3 may pass 2^24 by a quarter and a half, where the last
+// unit, 2^-40 and 2^-50 of the scales, may be lost.  Each sum is added to the FP64 result with its power-of-two
+// weight.  The error is the dropped slices: about 2^-40 of 2^(ea_i + eb_j) per term (FP64 rounding for the
 // rest), against 2^-24 for plain FP32 operands.
 // A 64 x 64 output tile per workgroup: wave w computes the 32 x 32 quarter at rows 32 (w / 2),
-// columns 32 (w % 2) as 2 x 2 blocks of 16 x 16.
-// MFMA lane layout (16x16x4): A[i][k] from lane i + 16 k, B[k][j] from lane j + 16 k,
+// columns 32 (w % 2) as 2 x 2 blocks of 16 x 16.  Every thread splits eight consecutive K of one row of op(A) and
+// of one column of op(B) per stage of two chunks, loaded a stage ahead, and stores each slice's fours as 8-byte words,
+// the words a lane of the matrix cores takes: A[i][4 g .. 4 g + 3] from lane i + 16 g, B likewise,
 // D[4 (l / 16) + v][l % 16] in element v of lane l.
+// (The slices as FP32 on v_mfma_f32_16x16x4f32, 40 of those and ten sums per chunk and block where there are ten
+// and four now: the two products of an update of 512 rows and ranks near 190 took 3.6 ms in one workgroup, 0.8 now,
+// with the same errors.)
 // ---------------------------------------------------------------------------
 constexpr int MS_BITS = 10, MS_SLICES = 4;
-constexpr int GTM_SLICE_A = GT_K * (GT_M + 1), GTM_SLICE_B = GT_K * (GT_N + 1);
-constexpr int GTM_LDS_FLOATS = MS_SLICES * (GTM_SLICE_A + GTM_SLICE_B) + GT_M + GT_N;
+constexpr int MS_KC = 2 * GT_K;                  // K staged at a time: two chunks per round trip and barrier pair
+constexpr int MS_KT = MS_KC / 4;                 // of which a thread splits these for one row and one column
+constexpr int MS_LD = MS_KC + 4;                 // halves per row of a slice: 8-byte words, banks spread
+constexpr int MS_SLICE = GT_M * MS_LD;           // halves per slice of either operand
+constexpr int GTM_LDS_FLOATS = MS_SLICES * MS_SLICE + GT_M + GT_N;
+static_assert(GT_M == GT_N && GT_K == 16 && GT_M * 4 == NT, "a thread per row and four K");
 static_assert(2 * MS_BITS + 4 <= 24, "slice products over a 16-deep chunk must be exact in FP32");
 
-// Slices of v in [-1, 1] (a value divided by its row's or column's power-of-two scale).
-__device__ __forceinline__ void ms_split(double v, float (&x)[MS_SLICES]) {
-    double r = v;
-#pragma unroll
-    for (int s = 0; s < MS_SLICES; ++s) {
-        const double q = rint(ldexp(r, MS_BITS * (s + 1)));
-        x[s] = (float) q;
-        r -= ldexp(q, -MS_BITS * (s + 1));
-    }
-}
+typedef _Float16 hcamd_halfx4 __attribute__((ext_vector_type(4)));
 
 // Exponent e with |v| < 2^e for the largest magnitude v of a row or column (0 for a zero one).
 __device__ __forceinline__ int ms_exponent(double vmax) {
     return vmax > 0.0 ? ilogb(vmax) + 1 : 0;
 }
 
+// Slices of MS_KT values in [-1, 1] (divided by their row's or column's power-of-two scale), each slice's
+// stored at dst + s MS_SLICE.
+__device__ __forceinline__ void ms_split(const double (&v)[MS_KT], int e, _Float16 *dst) {
+#pragma unroll
+    for (int k0 = 0; k0 < MS_KT; k0 += 4) {
+        float x[MS_SLICES][4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            double r = ldexp(v[k0 + k], MS_BITS - e);
+#pragma unroll
+            for (int s = 0; s < MS_SLICES; ++s) {
+                const double q = rint(r);
+                x[s][k] = (float) q;
+                r = (r - q) * double(1 << MS_BITS);
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < MS_SLICES; ++s) {
+            // packed conversions (exact here); a cast of a rounded double to _Float16 becomes a software conversion
+            const auto lo = __builtin_amdgcn_cvt_pkrtz(x[s][0], x[s][1]), hi = __builtin_amdgcn_cvt_pkrtz(x[s][2], x[s][3]);
+            uint2 u;
+            __builtin_memcpy(&u.x, &lo, 4);
+            __builtin_memcpy(&u.y, &hi, 4);
+            *reinterpret_cast<uint2 *>(dst + s * MS_SLICE + k0) = u;
+        }
+    }
+}
+
 __device__ inline void wg_gemm_tile_mixed(int M, int N, int Kd, const double *A, int64_t lda, bool ta,
                                           const double *B, int64_t ldb, bool tb, double *C, int64_t ldc, int ti,
                                           int tj, float *lds) {
-    float *As = lds;                                   // [slice][k][i], GTM_SLICE_A per slice
-    float *Bs = lds + MS_SLICES * GTM_SLICE_A;         // [slice][k][j]
-    int *ea = reinterpret_cast<int *>(Bs + MS_SLICES * GTM_SLICE_B);  // row exponents of op(A)
-    int *eb = ea + GT_M;                                               // column exponents of op(B)
-    const int i0 = ti * GT_M, j0 = tj * GT_N;
-    const int l = lane_id(), w = wave_id();
-    const int wr = 32 * (w / 2), wc = 32 * (w % 2);
-    auto opA = [&](int i, int k) -> double { return ta ? A[k + (int64_t) i * lda] : A[i + (int64_t) k * lda]; };
-    auto opB = [&](int k, int j) -> double { return tb ? B[j + (int64_t) k * ldb] : B[k + (int64_t) j * ldb]; };
-    // power-of-two scales: four threads per row of op(A) (then per column of op(B)) scan K
-    {
-        const int idx = threadIdx.x / 4, part = threadIdx.x % 4;
-        double amax = 0.0, bmax = 0.0;
-        if (i0 + idx < M)
-            for (int k = part; k < Kd; k += 4) amax = fmax(amax, fabs(opA(i0 + idx, k)));
-        if (j0 + idx < N)
-            for (int k = part; k < Kd; k += 4) bmax = fmax(bmax, fabs(opB(k, j0 + idx)));
-        amax = fmax(amax, __shfl_xor(amax, 1, WAVE));
-        amax = fmax(amax, __shfl_xor(amax, 2, WAVE));
-        bmax = fmax(bmax, __shfl_xor(bmax, 1, WAVE));
-        bmax = fmax(bmax, __shfl_xor(bmax, 2, WAVE));
-        if (part == 0) {
-            ea[idx] = ms_exponent(amax);
-            eb[idx] = ms_exponent(bmax);
+    _Float16 *As = reinterpret_cast<_Float16 *>(lds);  // [slice][i][k]
+    _Float16 *Bs = As + MS_SLICES * MS_SLICE;          // [slice][j][k]
+    int *ea = reinterpret_cast<int *>(Bs + MS_SLICES * MS_SLICE);  // row exponents of op(A)
+    int *eb = ea + GT_M;                                           // column exponents of op(B)
+    const int l = lane_id(), w = wave_id(), t = (int) threadIdx.x;
+    const int wr = 32 * (w / 2), wc = 32 * (w % 2), i16 = l & 15, g = l >> 4;
+    // this thread's row of op(A) and column of op(B), and its K of every stage: along the memory order
+    const int ai = ta ? t / 4 : t % GT_M, ak = MS_KT * (ta ? t % 4 : t / GT_M);
+    const int bj = tb ? t % GT_N : t / 4, bk = MS_KT * (tb ? t / GT_N : t % 4);
+    const int gi = ti * GT_M + ai, gj = tj * GT_N + bj;
+    const double *pa = A + (gi < M ? (ta ? gi * lda : gi) : 0), *pb = B + (gj < N ? (tb ? gj : gj * ldb) : 0);
+    const int64_t sa = ta ? 1 : lda, sb = tb ? ldb : 1;
+    auto load_one = [&](const double *p, int64_t st, int left, double (&x)[MS_KT]) {
+        if (left >= MS_KT) {
+#pragma unroll
+            for (int s = 0; s < MS_KT; ++s) x[s] = p[s * st];
+        } else {
+#pragma unroll
+            for (int s = 0; s < MS_KT; ++s) x[s] = s < left ? p[s * st] : 0.0;
         }
+    };
+    auto load = [&](int k0, double (&a)[MS_KT], double (&b)[MS_KT]) {
+        load_one(pa + (k0 + ak) * sa, sa, gi < M ? Kd - k0 - ak : 0, a);
+        load_one(pb + (k0 + bk) * sb, sb, gj < N ? Kd - k0 - bk : 0, b);
+    };
+    // power-of-two scales: every thread's share of its row and column, then the four shares' largest
+    {
+        double amax = 0.0, bmax = 0.0;
+#pragma unroll 2
+        for (int k0 = 0; k0 < Kd; k0 += MS_KC) {
+            double a[MS_KT], b[MS_KT];
+            load(k0, a, b);
+#pragma unroll
+            for (int s = 0; s < MS_KT; ++s) {
+                amax = fmax(amax, fabs(a[s]));
+                bmax = fmax(bmax, fabs(b[s]));
+            }
+        }
+        double *red = reinterpret_cast<double *>(lds);
+        red[ai + GT_M * (ak / MS_KT)] = amax;
+        red[NT + bj + GT_N * (bk / MS_KT)] = bmax;
+        __syncthreads();
+        if (t < GT_M + GT_N) {
+            const double *r = red + (t < GT_M ? t : NT + t - GT_M);
+            ea[t] = ms_exponent(fmax(fmax(r[0], r[GT_M]), fmax(r[2 * GT_M], r[3 * GT_M])));
+        }
+        __syncthreads();
     }
+    const int ae = ea[ai], be = eb[bj];
     double acc[2][2][4];
 #pragma unroll
     for (int p = 0; p < 2; ++p)
@@ -343,71 +395,44 @@ __device__ inline void wg_gemm_tile_mixed(int M, int N, int Kd, const double *A,
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v) acc[p][q][v] = 0.0;
-    __syncthreads();
-    for (int k0 = 0; k0 < Kd; k0 += GT_K) {
-        for (int e = threadIdx.x; e < GT_M * GT_K; e += NT) {
-            int i, k;
-            if (ta) {
-                k = e % GT_K;
-                i = e / GT_K;
-            } else {
-                i = e % GT_M;
-                k = e / GT_M;
-            }
-            const int gi = i0 + i, gk = k0 + k;
-            const double v = (gi < M && gk < Kd) ? ldexp(opA(gi, gk), -ea[i]) : 0.0;
-            float x[MS_SLICES];
-            ms_split(v, x);
-#pragma unroll
-            for (int sl = 0; sl < MS_SLICES; ++sl) As[sl * GTM_SLICE_A + k * (GT_M + 1) + i] = x[sl];
-        }
-        for (int e = threadIdx.x; e < GT_N * GT_K; e += NT) {
-            int j, k;
-            if (tb) {
-                j = e % GT_N;
-                k = e / GT_N;
-            } else {
-                k = e % GT_K;
-                j = e / GT_K;
-            }
-            const int gj = j0 + j, gk = k0 + k;
-            const double v = (gj < N && gk < Kd) ? ldexp(opB(gk, gj), -eb[j]) : 0.0;
-            float x[MS_SLICES];
-            ms_split(v, x);
-#pragma unroll
-            for (int sl = 0; sl < MS_SLICES; ++sl) Bs[sl * GTM_SLICE_B + k * (GT_N + 1) + j] = x[sl];
-        }
+    double na[MS_KT], nb[MS_KT];
+    load(0, na, nb);
+    for (int k0 = 0; k0 < Kd; k0 += MS_KC) {
+        ms_split(na, ae, As + ai * MS_LD + ak);
+        ms_split(nb, be, Bs + bj * MS_LD + bk);
         __syncthreads();
+        if (k0 + MS_KC < Kd) load(k0 + MS_KC, na, nb);
 #pragma unroll
-        for (int sa = 0; sa < MS_SLICES; ++sa) {
+        for (int c = 0; c < MS_KC; c += GT_K) {
+            if (k0 + c >= Kd) break;
+            hcamd_halfx4 a[2][MS_SLICES], b[2][MS_SLICES];
 #pragma unroll
-            for (int sb = 0; sb + sa < MS_SLICES; ++sb) {
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int s = 0; s < MS_SLICES; ++s) {
+                    const int o = s * MS_SLICE + (16 * p + i16) * MS_LD + c + 4 * g;
+                    __builtin_memcpy(&a[p][s], __builtin_assume_aligned(As + wr * MS_LD + o, 8), 8);
+                    __builtin_memcpy(&b[p][s], __builtin_assume_aligned(Bs + wc * MS_LD + o, 8), 8);
+                }
+#pragma unroll
+            for (int d = 0; d < MS_SLICES; ++d) {
                 hcamd_floatx4 part[2][2];
 #pragma unroll
                 for (int p = 0; p < 2; ++p)
 #pragma unroll
-                    for (int q = 0; q < 2; ++q) part[p][q] = hcamd_floatx4{0.f, 0.f, 0.f, 0.f};
+                    for (int q = 0; q < 2; ++q) {
+                        part[p][q] = hcamd_floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int kk = 0; kk < GT_K; kk += 4) {
-                    const int k = kk + l / 16;
-                    float a[2], b[2];
-#pragma unroll
-                    for (int p = 0; p < 2; ++p) a[p] = As[sa * GTM_SLICE_A + k * (GT_M + 1) + wr + 16 * p + (l % 16)];
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) b[q] = Bs[sb * GTM_SLICE_B + k * (GT_N + 1) + wc + 16 * q + (l % 16)];
-#pragma unroll
-                    for (int p = 0; p < 2; ++p)
-#pragma unroll
-                        for (int q = 0; q < 2; ++q)
-                            part[p][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[p], b[q], part[p][q], 0, 0, 0);
-                }
-                const double wgt = ldexp(1.0, -MS_BITS * (sa + sb + 2));
+                        for (int s = 0; s <= d; ++s)
+                            part[p][q] = __builtin_amdgcn_mfma_f32_16x16x16f16(a[p][s], b[q][d - s], part[p][q], 0, 0, 0);
+                    }
+                const double wgt = 1.0 / double(int64_t(1) << (MS_BITS * (d + 2)));
 #pragma unroll
                 for (int p = 0; p < 2; ++p)
 #pragma unroll
                     for (int q = 0; q < 2; ++q)
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) acc[p][q][v] += (double) part[p][q][v] * wgt;
+                        for (int v = 0; v < 4; ++v) acc[p][q][v] = fma((double) part[p][q][v], wgt, acc[p][q][v]);
             }
         }
         __syncthreads();
@@ -418,9 +443,9 @@ __device__ inline void wg_gemm_tile_mixed(int M, int N, int Kd, const double *A,
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int ri = wr + 16 * p + 4 * (l / 16) + v, cj = wc + 16 * q + (l % 16);
-                const int gi = i0 + ri, gj = j0 + cj;
-                if (gi < M && gj < N) C[gi + (int64_t) gj * ldc] = ldexp(acc[p][q][v], ea[ri] + eb[cj]);
+                const int ri = wr + 16 * p + 4 * g + v, cj = wc + 16 * q + i16;
+                const int ci = ti * GT_M + ri, cc = tj * GT_N + cj;
+                if (ci < M && cc < N) C[ci + (int64_t) cc * ldc] = ldexp(acc[p][q][v], ea[ri] + eb[cj]);
             }
     __syncthreads();
 }

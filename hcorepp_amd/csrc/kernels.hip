@@ -588,7 +588,7 @@ __global__ void HCAMD_KERNEL k_readjust_ddc(const T *W, int64_t m, int64_t n, T 
 // ---------------------------------------------------------------------------
 static_assert(GTM_LDS_FLOATS * sizeof(float) <= (size_t) BATCH_LDS_BYTES, "mixed tile GEMM LDS");
 
-// Factor products of one update (C.Gemm's temporaries).  mixed: FP32 matrix-core products of
+// Factor products of one update (C.Gemm's temporaries).  mixed: FP16 matrix-core products of
 // the operands' error-free slices with FP32 accumulation (FP64 operands and results,
 // wg_gemm_mixed), otherwise FP64.
 template <typename T>

@@ -48,8 +48,8 @@ typedef enum { HCOREPP_SVD_GESVD = 0, HCOREPP_SVD_GESDD = 1 } hcorepp_svd_type;
 /* Precision form of a batch (north-star forms). */
 typedef enum {
     HCOREPP_PREC_FP64 = 0,   /* everything in FP64 */
-    HCOREPP_PREC_MIXED = 1   /* factor products (the temporary tiles of HCore.cpp:176-264) on the FP32
-                                matrix cores with FP32 accumulation; stacking, both QRs, the core SVD, the
+    HCOREPP_PREC_MIXED = 1   /* factor products (the temporary tiles of HCore.cpp:176-264) on the FP16
+                                matrix cores over exact slices of the FP64 operands, FP32 accumulation; stacking, both QRs, the core SVD, the
                                 truncation decision and the reconstruction in FP64 */
 } hcorepp_precision;
 
