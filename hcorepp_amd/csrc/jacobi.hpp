@@ -402,19 +402,22 @@ __device__ __forceinline__ int wg_gram_jacobi(T *J, int64_t ldj, int rows, int n
 
 // Jacobi without V for a core too large for LDS, staged through it by super-blocks, by one workgroup
 // of NWAVES waves, NS of them per tile.  The columns form super-blocks of W = GJ_B * NWAVES / NS
-// columns and each sweep runs the round-robin ordering over super-blocks.  For a super-block pair
-// (SI, SJ), both are copied into the LDS buffer Jl (ld rows | 1; SI in local columns [0, W), SJ in
-// [W, 2 W), columns past ncols zero, so they never rotate), the waves rotate its block pairs
-// there round by round, and the pair is copied back.  In the first super-step every super-block
-// appears once, and its pair runs the round-robin over all 2 W / GJ_B local blocks (in whose first round
-// each block appears once, as a full tile: its internal column pairs); later super-steps visit only
-// the block pairs across SI and SJ, W / GJ_B rounds.  So every column pair is visited once per sweep, as in
-// wg_gram_jacobi, while the core passes through memory once per super-step instead of once per
-// block step.  J: rows x ncols (ld rows); lds: gram_jacobi_lds<T>(NWAVES) elements of LDS, Jl: 2 W (rows | 1).
+// columns and each sweep visits the super-block pairs (I, J > I) row by row: SI stays in local columns [0, W) of the
+// LDS buffer Jl (ld rows | 1) while SJ after SJ passes through [W, 2 W), the next one on its way into
+// registers as the waves rotate the block pairs of this one, round by round.  (One workgroup does them one
+// after the other, so nothing asks for the disjoint pairs of a round-robin, which copied both super-blocks in and
+// out per pair.  At 128 to 160 columns, two workgroups per CU: 647 us per sweep and 5.8 sweeps then, 617 and
+// 5.1 now, since later pairs meet columns that earlier ones have turned; beyond, 1195 and 5.6, 1130 and 5.2.)
+// The pairs (0, 1), (2, 3), ... run the round-robin over all their 2 W / GJ_B local blocks (in whose first round
+// each block appears once, as a full tile: its internal column pairs), the others only the block pairs across SI and
+// SJ, W / GJ_B rounds.  So every column pair is visited once per sweep, as in wg_gram_jacobi.  Columns past
+// ncols are zero, so they never rotate.  A thread moves the same elements of a super-block wherever it goes,
+// so the copies need no barrier among themselves.
+// J: rows x ncols (ld rows), rows <= 64 RC; lds: gram_jacobi_lds<T>(NWAVES) elements of LDS, Jl: 2 W (rows | 1).
 // Returns the sweeps used.
-template <typename T, int NS>
+template <typename T, int NS, int RC>
 __device__ __forceinline__ int wg_staged_jacobi(T *J, int rows, int ncols, T *Jl, T stop, int max_sweeps, T *lds) {
-    constexpr int A = NWAVES / NS, W = GJ_B * A, LC = 2 * W;
+    constexpr int A = NWAVES / NS, W = GJ_B * A, LC = 2 * W, CW = W / NWAVES;
     T *s_red = lds;
     int &s_rot = *reinterpret_cast<int *>(lds + 8);
     T *sc = lds + 16 + wave_id() * GJ_SC;
@@ -428,51 +431,50 @@ __device__ __forceinline__ int wg_staged_jacobi(T *J, int rows, int ncols, T *Jl
     const GramTol<T> g(wg_sum(part, s_red), rows, stop);
     if (ncols <= 1) return 0;
     const int ld = rows | 1;
-    const int ns = (ncols + W - 1) / W, nsp = ns + (ns & 1);
-    // the pair's columns between memory (ld rows) and LDS (ld `ld`): a wave takes every NWAVES-th
-    // column, all of them in flight together per 64 rows
-    constexpr int CPW = LC / NWAVES;
-    auto load = [&](int cI, int nI, int cJ, int nJ) {
-        for (int r = lane_id(); r < rows; r += WAVE) {
-            T v[CPW];
+    const int ns = (ncols + W - 1) / W;
+    // super-block S between memory (ld rows), registers and local columns [c0, c0 + W): a wave takes every
+    // NWAVES-th column, a lane every 64th row
+    T next[RC][CW];
+    auto each = [&](int S, int c0, auto &&f) {
 #pragma unroll
-            for (int u = 0; u < CPW; ++u) {
-                const int c = wave_id() + u * NWAVES;
-                const int gc = c < W ? (c < nI ? cI + c : -1) : (c - W < nJ ? cJ + c - W : -1);
-                v[u] = gc >= 0 ? J[r + (int64_t) gc * rows] : T(0);
+        for (int t = 0; t < RC; ++t)
+#pragma unroll
+            for (int u = 0; u < CW; ++u) {
+                const int r = lane_id() + WAVE * t, c = wave_id() + u * NWAVES;
+                f(t, u, J + r + (int64_t) (S * W + c) * rows, Jl + r + (c0 + c) * ld, r < rows, S * W + c < ncols);
             }
-#pragma unroll
-            for (int u = 0; u < CPW; ++u) Jl[r + (wave_id() + u * NWAVES) * ld] = v[u];
-        }
     };
-    auto store = [&](int cI, int nI, int cJ, int nJ) {
-        for (int r = lane_id(); r < rows; r += WAVE) {
-            T v[CPW];
-#pragma unroll
-            for (int u = 0; u < CPW; ++u) v[u] = Jl[r + (wave_id() + u * NWAVES) * ld];
-#pragma unroll
-            for (int u = 0; u < CPW; ++u) {
-                const int c = wave_id() + u * NWAVES;
-                const int gc = c < W ? (c < nI ? cI + c : -1) : (c - W < nJ ? cJ + c - W : -1);
-                if (gc >= 0) J[r + (int64_t) gc * rows] = v[u];
-            }
-        }
+    auto fetch = [&](int S) {
+        each(S, 0, [&](int t, int u, const T *m, T *, bool row, bool col) { next[t][u] = row && col ? *m : T(0); });
+    };
+    auto put = [&](int c0) {
+        each(0, c0, [&](int t, int u, T *, T *q, bool row, bool) {
+            if (row) *q = next[t][u];
+        });
+    };
+    auto save = [&](int S, int c0) {
+        each(S, c0, [&](int, int, T *m, const T *q, bool row, bool col) {
+            if (row && col) *m = *q;
+        });
     };
     int sweep = 0;
     for (; sweep < max_sweeps; ++sweep) {
         if (threadIdx.x == 0) s_rot = 0;
         __syncthreads();
         int any = 0;
-        for (int ss = 0; ss < nsp - 1; ++ss) {
-            for (int sp = 0; sp < nsp / 2; ++sp) {
-                int cI, cJ;
-                if (!jacobi_pair_cols(sp, ss, nsp, W, ncols, cI, cJ)) continue;
-                const bool solo = cJ >= ncols;  // paired with the padding super-block
-                if (ss > 0 && solo) continue;
-                const int nI = (ncols - cI) < W ? (ncols - cI) : W;
-                const int nJ = solo ? 0 : ((ncols - cJ) < W ? (ncols - cJ) : W);
-                load(cI, nI, cJ, nJ);
+        for (int I = 0; I < ns; ++I) {
+            // the last super-block has no partner: alone, only if no pair has visited its inside
+            const bool solo = I == ns - 1;
+            if (solo && (I & 1)) break;
+            fetch(I);
+            put(0);
+            fetch(I + 1);  // zeros past the end
+            const int nI = (ncols - I * W) < W ? (ncols - I * W) : W;
+            for (int S = I + 1; S < ns || (solo && S == ns); ++S) {
+                put(W);
                 __syncthreads();
+                if (S + 1 < ns) fetch(S + 1);
+                const int left = ncols - S * W, nJ = left < 0 ? 0 : (left < W ? left : W);
                 // a tile is skipped when no pair of it can rotate (a cross tile with an empty block, a
                 // full tile with two)
                 auto real = [&](int lc) { return lc < W ? lc < nI : lc - W < nJ; };
@@ -481,26 +483,19 @@ __device__ __forceinline__ int wg_staged_jacobi(T *J, int rows, int ncols, T *Jl
                     const bool act = full ? (real(lI) || real(lJ)) : (real(lI) && real(lJ));
                     if (NS > 1 || act) rot |= gram_tile<T, NS>(act, Jl, ld, rows, LC, lI, lJ, full, g, sc, sub);
                 };
-                if (ss == 0) {
-                    // the round-robin over the local blocks: all 2 A of them
-                    for (int t = 0; t < 2 * A - 1; ++t) {
-                        int lI, lJ;
-                        jacobi_pair_cols(grp, t, 2 * A, GJ_B, LC, lI, lJ);
-                        visit(lI, lJ, t == 0);
-                        __syncthreads();
-                    }
-                } else {
-                    for (int t = 0; t < A; ++t) {
-                        int q = grp + t;
-                        if (q >= A) q -= A;
-                        visit(grp * GJ_B, W + q * GJ_B, false);
-                        __syncthreads();
-                    }
+                // the round-robin over the local blocks, all 2 A of them, or those across
+                const bool inside = S == I + 1 && !(I & 1);
+                const int rounds = inside ? 2 * A - 1 : A;
+                for (int t = 0; t < rounds; ++t) {
+                    int lI = grp * GJ_B, lJ = W + (grp + t < A ? grp + t : grp + t - A) * GJ_B;
+                    if (inside) jacobi_pair_cols(grp, t, 2 * A, GJ_B, LC, lI, lJ);
+                    visit(lI, lJ, inside && t == 0);
+                    __syncthreads();
                 }
                 any |= rot;
-                store(cI, nI, cJ, nJ);
-                __syncthreads();
+                if (S < ns) save(S, W);
             }
+            save(I, 0);
         }
         if ((any & JROT_LARGE) && lane_id() == 0) atomicOr(&s_rot, 1);
         __syncthreads();
@@ -508,6 +503,7 @@ __device__ __forceinline__ int wg_staged_jacobi(T *J, int rows, int ncols, T *Jl
         __syncthreads();
         if (!rot) break;
     }
+    __syncthreads();
     return sweep;
 }
 

@@ -1330,8 +1330,9 @@ template <typename T, int NS>
 __device__ HCAMD_PHASE_ATTR int jacobi_nov_staged(T *J, int rows, int ncols) {
     extern __shared__ unsigned char smem_raw[];
     T *lds = reinterpret_cast<T *>(smem_raw);
-    return wg_staged_jacobi<T, NS>(J, rows, ncols, lds + gram_jacobi_lds<T>(NWAVES), JacobiStopCos<T>::loose,
-                                   JACOBI_MAX_SWEEPS, lds);
+    constexpr int RC = (int) (nov_lds_cap<T>() / (2 * GJ_B * NWAVES / NS) + WAVE - 1) / WAVE;
+    return wg_staged_jacobi<T, NS, RC>(J, rows, ncols, lds + gram_jacobi_lds<T>(NWAVES), JacobiStopCos<T>::loose,
+                                       JACOBI_MAX_SWEEPS, lds);
 }
 
 template <typename T>
