@@ -111,19 +111,19 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_qr_panel(PlainQr<T> q, RecompDe
     });
 }
 
-// Trailing update: workgroup x takes the columns at positions j0 + jb + 16 x .. + 15.  The block is read
+// Trailing update: workgroup x takes the uc <= 16 columns at positions j0 + jb + uc x on.  The block is read
 // once, kept in registers through both products and written back; pivoted, its rows of R go to J and the
 // squared norms below them to cn for the next panel's pivoting.
 template <typename T, int WAVES, int GROUPS>
-__global__ void __launch_bounds__(WAVES *WAVE) k_qr_update(PlainQr<T> q, int j0) {
+__global__ void __launch_bounds__(WAVES *WAVE) k_qr_update(PlainQr<T> q, int j0, int uc) {
     __shared__ WyLds<T, WAVES> lds;
     using MF = Mfma16<T>;
     const int ln = lane_id(), i16 = ln & 15, k4 = ln >> 4, wv = wave_id();
     const int rows = q.m - j0;
     const int nsteps = q.m < q.ncols ? q.m : q.ncols;
     const int jb = nsteps - j0 < PQ_NB ? nsteps - j0 : PQ_NB;
-    const int pos = j0 + jb + PQ_NB * (int) blockIdx.x + i16;
-    const bool cok = pos < q.ncols, wide = wide_columns(q.A, q.m);
+    const int pos = j0 + jb + uc * (int) blockIdx.x + i16;
+    const bool cok = i16 < uc && pos < q.ncols, wide = wide_columns(q.A, q.m);
     auto column = [&](int p) { return q.pivot ? q.piv[p] : p; };
     const int c = column(cok ? pos : j0);
     const T *pcol = q.A + (int64_t) column(j0 + (i16 < jb ? i16 : 0)) * q.m + j0;
@@ -210,9 +210,12 @@ static hipError_t launch_qr(hipStream_t s, const RecompDesc<T> &d, const PlainQr
         pq_shape(q.m - j0, [&](auto waves, auto groups) {
             constexpr int WV = decltype(waves)::value, GR = decltype(groups)::value;
             hipLaunchKernelGGL((k_qr_panel<T, WV, GR>), dim3(1), dim3(WV * WAVE), 0, s, q, d, kk, j0);
+            // four columns per workgroup while that is one workgroup per CU at most: an update is bound by what one CU
+            // moves of its columns, not by the matrix cores, which 16 would fill (1024 rows 24.8 us with 16, 20.9 with
+            // 8, 19.0 with 4; 512 rows 13.8, 11.9, 11.0; 256 rows 8.4, 7.6, 7.1)
+            const int uc = trail <= 4 * 256 ? 4 : PQ_NB;
             if (trail > 0)
-                hipLaunchKernelGGL((k_qr_update<T, WV, GR>), dim3((trail + PQ_NB - 1) / PQ_NB), dim3(WV * WAVE), 0, s, q,
-                                   j0);
+                hipLaunchKernelGGL((k_qr_update<T, WV, GR>), dim3((trail + uc - 1) / uc), dim3(WV * WAVE), 0, s, q, j0, uc);
         });
     }
     return hipGetLastError();
