@@ -40,3 +40,17 @@ def test_block_edges(ctx, m, n, ra, rc, dtype, eps):
     good = sig[: u.shape[1]] > 1e3 * eps * sig[0]
     g = u[:, good].T @ u[:, good]
     assert np.abs(g - np.eye(len(g))).max() < 100 * (ra + rc + 1) * eps
+
+
+@pytest.mark.parametrize("ra,rc", [(520, 520), (520, 521), (530, 530)])
+def test_more_stacked_columns_than_one_launch_row(ctx, ra, rc):
+    """Stacked ranks on either side of 1040, where the first trailing updates go from 4 columns per workgroup to 16; the
+    result has full rank, so nothing is truncated.  Bound as above."""
+    import hcorepp_amd as H
+    rng = np.random.default_rng(ra + 3 * rc)
+    m, n, k = 600, 560, 540
+    a, b, c = _pair(rng, m, k, ra), _pair(rng, k, n, ra), _pair(rng, m, n, rc)
+    full = c[0] @ c[1] + (a[0] @ a[1]) @ (b[0] @ b[1])
+    C = H.CompressedTile(*c, max_rank=n)
+    H.HCore.gemm(1.0, H.CompressedTile(*a), H.CompressedTile(*b), 1.0, C, ctx, H.CompressionParameters(1e-14))
+    assert rel_fro(C.to_dense(), full) < 100 * (ra + rc + 1) * 2.2e-16
