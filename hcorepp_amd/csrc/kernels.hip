@@ -117,7 +117,6 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_qr_panel(PlainQr<T> q, RecompDe
 template <typename T, int WAVES, int GROUPS>
 __global__ void __launch_bounds__(WAVES *WAVE) k_qr_update(PlainQr<T> q, int j0, int uc) {
     __shared__ WyLds<T, WAVES> lds;
-    using MF = Mfma16<T>;
     const int ln = lane_id(), i16 = ln & 15, k4 = ln >> 4, wv = wave_id();
     const int rows = q.m - j0;
     const int nsteps = q.m < q.ncols ? q.m : q.ncols;
@@ -127,19 +126,12 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_qr_update(PlainQr<T> q, int j0,
     auto column = [&](int p) { return q.pivot ? q.piv[p] : p; };
     const int c = column(cok ? pos : j0);
     const T *pcol = q.A + (int64_t) column(j0 + (i16 < jb ? i16 : 0)) * q.m + j0;
-    const T *prow[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const int k = MF::row(s, k4);
-        prow[s] = q.A + (int64_t) column(j0 + (k < jb ? k : 0)) * q.m + j0;
-    }
     if (q.pivot && q.hdr[HDR_KQ] > 0) return;  // the QR of Y stopped early
     T *col = q.A + (int64_t) c * q.m + j0;
     T b[GROUPS][4];
 #pragma unroll
     for (int t = 0; t < GROUPS; ++t) load_rows(col, 16 * (wv + WAVES * t) + 4 * k4, rows, cok, wide, b[t]);
     const T *ts = q.tsave + (int64_t) (j0 / PQ_NB) * PQ_NB * PQ_NB;
-    const int pr = pq_prow<T>(i16);
     // the panel's columns hold R on and above the diagonal: unit lower in the first group of rows
     wy_block<T, WAVES, GROUPS>(
             b,
@@ -153,11 +145,6 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_qr_update(PlainQr<T> q, int j0,
                         v[s] = r > i16 ? v[s] : T(r == i16 && i16 < jb);
                     }
                 }
-            },
-            [&](int t, int s) {
-                const int r = 16 * (wv + WAVES * t) + pr, k = MF::row(s, k4);
-                if (k >= jb || r >= rows || r < k) return T(0);
-                return r == k ? T(1) : prow[s][r];
             },
             [&](int i, int j) { return i <= j ? ts[i + PQ_NB * j] : T(0); }, true, 0, lds);
     T nsq = T(0);
@@ -212,7 +199,7 @@ static hipError_t launch_qr(hipStream_t s, const RecompDesc<T> &d, const PlainQr
             hipLaunchKernelGGL((k_qr_panel<T, WV, GR>), dim3(1), dim3(WV * WAVE), 0, s, q, d, kk, j0);
             // four columns per workgroup while that is one workgroup per CU at most: an update is bound by what one CU
             // moves of its columns, not by the matrix cores, which 16 would fill (1024 rows 24.8 us with 16, 20.9 with
-            // 8, 19.0 with 4; 512 rows 13.8, 11.9, 11.0; 256 rows 8.4, 7.6, 7.1)
+            // 8, 19.0 with 4; 512 rows 13.8, 11.9, 11.0; 256 rows 8.4, 7.6, 7.1; 17.9, 10.5 and 7.0 since P is read once)
             const int uc = trail <= 4 * 256 ? 4 : PQ_NB;
             if (trail > 0)
                 hipLaunchKernelGGL((k_qr_update<T, WV, GR>), dim3((trail + uc - 1) / uc), dim3(WV * WAVE), 0, s, q, j0, uc);
@@ -497,7 +484,6 @@ template <typename T, int WAVES, int GROUPS>
 __global__ void __launch_bounds__(WAVES *WAVE) k_recon(RecompDesc<T> d) {
     __shared__ WyLds<T, WAVES> lds;
     __shared__ int32_t cols[PQ_MAX_COLS];  // the columns that hold the reflectors
-    using MF = Mfma16<T>;
     Ws<T> w = ws_of(d);
     const Dims z = dims_of(d, w);
     const int r = (int) w.hdr[HDR_RANK], side = (int) blockIdx.y;
@@ -521,7 +507,6 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_recon(RecompDesc<T> d) {
     // [v1 sigma; 0] vanishes below row kt, where reflectors kt.. of Q_Y act as the identity (each is zero
     // above its own row), so only the first kt are applied
     const int nref = side ? (z.kt < z.kk ? z.kt : z.kk) : z.mu;
-    const int pr = pq_prow<T>(i16);
     const bool wide = wide_columns(A, rows);
     for (int i = threadIdx.x; i < nref; i += WAVES * WAVE) cols[i] = side ? w.piv[i] : i;
     __syncthreads();
@@ -529,9 +514,6 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_recon(RecompDesc<T> d) {
         const int j0 = p * PQ_NB, jb = nref - j0 < PQ_NB ? nref - j0 : PQ_NB;
         const T *ts = tsave + (int64_t) p * PQ_NB * PQ_NB;
         const T *pcol = A + (int64_t) cols[j0 + (i16 < jb ? i16 : 0)] * rows;
-        const T *prow[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) prow[s] = A + (int64_t) cols[j0 + (MF::row(s, k4) < jb ? MF::row(s, k4) : 0)] * rows;
         // the panel is unit lower from row j0 on (a multiple of 16: one mixed group)
         wy_block<T, WAVES, GROUPS>(
                 b,
@@ -545,11 +527,6 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_recon(RecompDesc<T> d) {
                             v[s] = rr > i16 ? v[s] : T(rr == i16 && i16 < jb);
                         }
                     }
-                },
-                [&](int t, int s) {
-                    const int row = 16 * (wv + WAVES * t) + pr, k = MF::row(s, k4);
-                    if (k >= jb || row >= rows || row < j0 + k) return T(0);
-                    return row == j0 + k ? T(1) : prow[s][row];
                 },
                 [&](int i, int jj) { return (i <= jj && jj < jb) ? ts[i + PQ_NB * jj] : T(0); }, false, p, lds);
     }

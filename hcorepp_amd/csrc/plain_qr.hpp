@@ -188,7 +188,7 @@ struct PanelLds {
 // Bound by the chain of a column: two reductions' latency, a reciprocal square root and a reciprocal, one
 // barrier: 0.7 us per column up to 512 rows.  Lanes along the columns need two exchanges per sum where a row
 // per lane took six for 16 values.  A whole panel of the pivoted QR takes 20 us at 256 rows and 36 at 1024
-// (50 and 47, for half as many columns, in LDS with a row per thread and four waves), its trailing update 8 and 25.
+// (50 and 47, for half as many columns, in LDS with a row per thread and four waves), its trailing update 7 and 18.
 template <typename T, int WAVES, int GROUPS>
 __device__ __forceinline__ T panel_factor(T (&p)[GROUPS][4], int jb, T *tau, PanelLds<T, WAVES> &l) {
     const int ln = lane_id(), i16 = ln & 15, k4 = ln >> 4, wv = wave_id();
@@ -410,16 +410,24 @@ __device__ __forceinline__ void wg_panel(const PlainQr<T> &q, int j0, PanelLds<T
 // LDS of a block-reflector application.
 template <typename T, int WAVES>
 struct WyLds {
-    T part[WAVES][PQ_NB * PQ_NB];
+    T part[WAVES][PQ_NB * (PQ_NB + 1)];  // per wave: a group of P in turn, then the wave's share of P^T b
     T w[PQ_NB * (PQ_NB + 1)];
 };
 
-// b <- (I - P op(T) P^T) b for a register block b, on the matrix cores; op(T) is T^T with `trans`.  pa(t, v) and
-// pb(t, s) give P in the two layouts, zero outside its rows: pa rows 16 G + 4 k4 .. + 3 of column i16, pb row
-// 16 G + prow of column row(s, k4), G = wave + WAVES t; groups below g0 are zero in P and skipped.  tm(i, j)
-// gives T.  Two barriers; every wave of the workgroup calls it.
-template <typename T, int WAVES, int GROUPS, typename PA, typename PB, typename TM>
-__device__ __forceinline__ void wy_block(T (&b)[GROUPS][4], const PA &pa, const PB &pb, const TM &tm, bool trans, int g0,
+// Memory row, within a group, of output row i of the update's matrix-core product, chosen so that element
+// v of lane (i16, k4) is row 4 k4 + v.
+template <typename T>
+__device__ __forceinline__ int pq_prow(int i) {
+    return sizeof(T) == 8 ? 4 * (i & 3) + (i >> 2) : i;
+}
+
+// b <- (I - P op(T) P^T) b for a register block b, on the matrix cores; op(T) is T^T with `trans`.  pa(t, v) gives
+// P, zero outside its rows: rows 16 G + 4 k4 .. + 3 of column i16, G = wave + WAVES t; groups below g0 are zero in P
+// and skipped.  tm(i, j) gives T.  Two barriers; every wave of the workgroup calls it.  The second product takes P
+// with its rows along the lanes, which each wave gets from its own LDS: reading both forms from memory, a CU moved
+// P twice (update of 1024 rows 19.0 us, 17.9 now; reconstruction of 1024 rows and rank 341 435 us, 365 now).
+template <typename T, int WAVES, int GROUPS, typename PA, typename TM>
+__device__ __forceinline__ void wy_block(T (&b)[GROUPS][4], const PA &pa, const TM &tm, bool trans, int g0,
                                          WyLds<T, WAVES> &l) {
     using MF = Mfma16<T>;
     const int ln = lane_id(), i16 = ln & 15, k4 = ln >> 4, wv = wave_id();
@@ -427,13 +435,21 @@ __device__ __forceinline__ void wy_block(T (&b)[GROUPS][4], const PA &pa, const 
 #pragma unroll
     for (int t = 0; t < GROUPS; ++t) pa(t, a[t]);
 #pragma unroll
-    for (int t = 0; t < GROUPS; ++t)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) c[t][s] = pb(t, s);
-#pragma unroll
     for (int s = 0; s < 4; ++s) {
         const int k = MF::row(s, k4);
         top[s] = trans ? tm(k, i16) : tm(i16, k);
+    }
+    T *tile = l.part[wv];
+    const int pr = pq_prow<T>(i16);
+#pragma unroll
+    for (int t = 0; t < GROUPS; ++t) {
+        if (wv + WAVES * t < g0) continue;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) tile[i16 * (PQ_NB + 1) + 4 * k4 + s] = a[t][s];
+        wave_fence();
+#pragma unroll
+        for (int s = 0; s < 4; ++s) c[t][s] = tile[MF::row(s, k4) * (PQ_NB + 1) + pr];
+        wave_fence();
     }
     typename MF::acc acc = MF::zero();
 #pragma unroll
@@ -464,13 +480,6 @@ __device__ __forceinline__ void wy_block(T (&b)[GROUPS][4], const PA &pa, const 
 #pragma unroll
         for (int v = 0; v < 4; ++v) b[t][v] -= d[v];
     }
-}
-
-// Memory row, within a group, of output row i of the update's matrix-core product, chosen so that element
-// v of lane (i16, k4) is row 4 k4 + v.
-template <typename T>
-__device__ __forceinline__ int pq_prow(int i) {
-    return sizeof(T) == 8 ? 4 * (i & 3) + (i >> 2) : i;
 }
 
 }  // namespace hcamd
