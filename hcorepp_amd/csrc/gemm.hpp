@@ -277,20 +277,20 @@ __host__ __device__ inline bool gemm_is_small(int64_t M, int64_t N) {
 // by a power of two 2^ea_i above its largest magnitude and cut into MS_SLICES slices: integers
 // x_s of at most MS_BITS bits with op(A)[i, k] = 2^ea_i sum_s x_s 2^(-MS_BITS (s+1)) + (a rest
 // below 2^(ea_i - MS_BITS MS_SLICES - 1)); each column of op(B) likewise.  FP16 holds every such integer
-// exactly (|x_0| <= 2^10, the later ones 2^9).  The products of the slice pairs with s + t = d are summed in FP32
-// over one 16-deep K chunk: for d = 0 and 1, which carry the result's leading bits, at most 2^24 and exact
-// in whatever order the matrix core sums; d = 2 and 3 may pass 2^24 by a quarter and a half, where the last
-// unit, 2^-40 and 2^-50 of the scales, may be lost.  Each sum is added to the FP64 result with its power-of-two
-// weight.  The error is the dropped slices: about 2^-40 of 2^(ea_i + eb_j) per term (FP64 rounding for the
-// rest), against 2^-24 for plain FP32 operands.
+// exactly (|x_0| <= 2^10, the later ones 2^9).  The products of the pairs (s, t) and (t, s) are summed in FP32 over one
+// 16-deep K chunk, at most 16 * 2 * 2^10 * 2^9 = 2^24 and so exact in whatever order the matrix core sums, and each of
+// the six sums with s + t < MS_SLICES is added to the FP64 result with its power-of-two weight.  (One sum for all pairs of
+// a weight passes 2^24 where there are three or four of them, and lost units of 2^-40.)  The error is the dropped
+// slices: about 2^-40 of 2^(ea_i + eb_j) per term (FP64 rounding for the rest), against 2^-24 for plain FP32
+// operands.
 // A 64 x 64 output tile per workgroup: wave w computes the 32 x 32 quarter at rows 32 (w / 2),
 // columns 32 (w % 2) as 2 x 2 blocks of 16 x 16.  Every thread splits eight consecutive K of one row of op(A) and
 // of one column of op(B) per stage of two chunks, loaded a stage ahead, and stores each slice's fours as 8-byte words,
 // the words a lane of the matrix cores takes: A[i][4 g .. 4 g + 3] from lane i + 16 g, B likewise,
 // D[4 (l / 16) + v][l % 16] in element v of lane l.
 // (The slices as FP32 on v_mfma_f32_16x16x4f32, 40 of those and ten sums per chunk and block where there are ten
-// and four now: the two products of an update of 512 rows and ranks near 190 took 3.6 ms in one workgroup, 0.8 now,
-// with the same errors.)
+// and six now: the two products of an update of 512 rows and ranks near 190 took 3.6 ms in one workgroup, 1.0 now,
+// with the same errors; four sums, one per weight, 0.8, but not exact.)
 // ---------------------------------------------------------------------------
 constexpr int MS_BITS = 10, MS_SLICES = 4;
 constexpr int MS_KC = 2 * GT_K;                  // K staged at a time: two chunks per round trip and barrier pair
@@ -299,7 +299,7 @@ constexpr int MS_LD = MS_KC + 4;                 // halves per row of a slice: 8
 constexpr int MS_SLICE = GT_M * MS_LD;           // halves per slice of either operand
 constexpr int GTM_LDS_FLOATS = MS_SLICES * MS_SLICE + GT_M + GT_N;
 static_assert(GT_M == GT_N && GT_K == 16 && GT_M * 4 == NT, "a thread per row and four K");
-static_assert(2 * MS_BITS + 4 <= 24, "slice products over a 16-deep chunk must be exact in FP32");
+static_assert(4 + 1 + MS_BITS + (MS_BITS - 1) <= 24, "two slice pairs over a 16-deep chunk must be exact in FP32");
 
 typedef _Float16 hcamd_halfx4 __attribute__((ext_vector_type(4)));
 
@@ -416,23 +416,21 @@ __device__ inline void wg_gemm_tile_mixed(int M, int N, int Kd, const double *A,
                 }
 #pragma unroll
             for (int d = 0; d < MS_SLICES; ++d) {
-                hcamd_floatx4 part[2][2];
-#pragma unroll
-                for (int p = 0; p < 2; ++p)
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        part[p][q] = hcamd_floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int s = 0; s <= d; ++s)
-                            part[p][q] = __builtin_amdgcn_mfma_f32_16x16x16f16(a[p][s], b[q][d - s], part[p][q], 0, 0, 0);
-                    }
                 const double wgt = 1.0 / double(int64_t(1) << (MS_BITS * (d + 2)));
 #pragma unroll
-                for (int p = 0; p < 2; ++p)
+                for (int s = 0; 2 * s <= d; ++s) {
+                    const int t = d - s;
 #pragma unroll
-                    for (int q = 0; q < 2; ++q)
+                    for (int p = 0; p < 2; ++p)
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) acc[p][q][v] = fma((double) part[p][q][v], wgt, acc[p][q][v]);
+                        for (int q = 0; q < 2; ++q) {
+                            hcamd_floatx4 part{0.f, 0.f, 0.f, 0.f};
+                            part = __builtin_amdgcn_mfma_f32_16x16x16f16(a[p][s], b[q][t], part, 0, 0, 0);
+                            if (s != t) part = __builtin_amdgcn_mfma_f32_16x16x16f16(a[p][t], b[q][s], part, 0, 0, 0);
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) acc[p][q][v] = fma((double) part[v], wgt, acc[p][q][v]);
+                        }
+                }
             }
         }
         __syncthreads();
