@@ -58,11 +58,13 @@ __device__ __forceinline__ T col_sum(T v) {
 
 // Largest value of the wave, in every lane.
 __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
-    auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    v = r[0] > r[1] ? r[0] : r[1];
-    r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    v = r[0] > r[1] ? r[0] : r[1];
     auto step = [&](unsigned o) { v = o > v ? o : v; };
+    auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    v = r[0];
+    step(r[1]);
+    r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = r[0];
+    step(r[1]);
     step(__builtin_amdgcn_mov_dpp((int) v, DPP_ROW_MIRROR, 0xF, 0xF, true));
     step(__builtin_amdgcn_mov_dpp((int) v, DPP_ROW_HALF_MIRROR, 0xF, 0xF, true));
     step(__builtin_amdgcn_mov_dpp((int) v, DPP_QUAD_XOR2, 0xF, 0xF, true));
@@ -293,46 +295,65 @@ __device__ __forceinline__ T pivot_norm_sum(const T *cn, int nt) {
     return wave_sum(sum);
 }
 
-// Ordering key of a squared norm, from its exponent and leading mantissa bits: at least 16, NaN (and
-// anything negative) lowest; the four low bits are free.
-__device__ __forceinline__ unsigned norm_key(double v) {
-    return v > 0.0 ? ((unsigned) __double2hiint(v) & ~15u) + 16u : 16u;
+// Ordering key of a squared norm: its bits, which order as the norms do, above 0 for "no column" and 1 for NaN, the lowest.
+__device__ __forceinline__ unsigned long long norm_key(double v) {
+    return v >= 0.0 ? (unsigned long long) __double_as_longlong(v) + 2u : 1u;
 }
-__device__ __forceinline__ unsigned norm_key(float v) { return v > 0.f ? (__float_as_uint(v) & ~15u) + 16u : 16u; }
+__device__ __forceinline__ unsigned norm_key(float v) { return v >= 0.f ? __float_as_uint(v) + 2u : 1u; }
+
+// Largest key of the wave, in every lane.
+__device__ __forceinline__ unsigned wave_max_key(unsigned k) { return wave_max_u32(k); }
+__device__ __forceinline__ unsigned long long wave_max_key(unsigned long long k) {
+    const unsigned hi = wave_max_u32((unsigned) (k >> 32));
+    const unsigned lo = wave_max_u32((unsigned) (k >> 32) == hi ? (unsigned) k : 0u);
+    return (unsigned long long) hi << 32 | lo;
+}
 
 // Window pivoting at a panel's start, by wave 0: the jb trailing columns of largest norm (cn[p], p in
-// [0, nt), squared, by position) go to the panel, in decreasing norm; the columns they displace take the
-// positions they leave.  l.piv[0..nt) holds the columns by position and is permuted, and piv with it.
-// Norms are compared by 16 leading mantissa bits (closer ones are as good as each other), the key's low bits
-// holding which of its up to 12 columns a lane means: a lane sorts its keys once, and each round takes
-// the largest head of the wave's lists.  (Rounds over the unsorted norms in full took 0.5 us each; a count
-// of the larger norms per column, 768 x 768 reads of LDS, 10 us in all.)
+// [0, nt), squared, by position) go to the panel, in decreasing norm, equal ones by position; the columns they displace
+// take the positions they leave.  l.piv[0..nt) holds the columns by position and is permuted, and piv with it.
+// A lane sorts its up to 12 columns once, and each round takes the largest head of the wave's lists.  (Rounds over
+// the unsorted norms took 0.5 us each; a count of the larger norms per column, 768 x 768 reads of LDS, 10 us in all.)
 template <typename T, int WAVES, int PER>
 __device__ __forceinline__ void pivot_select(const T *cn, int nt, int jb, int32_t *piv, PanelLds<T, WAVES> &l) {
+    using Key = decltype(norm_key(T(0)));
     const int ln = lane_id();
-    unsigned key[PER];
+    Key key[PER];
+    int col[PER];
 #pragma unroll
     for (int t = 0; t < PER; ++t) {
-        const int c = ln + WAVE * t;
-        key[t] = c < nt ? norm_key(cn[c]) + t : 0u;
+        col[t] = ln + WAVE * t;
+        key[t] = col[t] < nt ? norm_key(cn[col[t]]) : Key(0);
     }
 #pragma unroll
     for (int ph = 0; ph < PER; ++ph)
 #pragma unroll
         for (int t = ph & 1; t + 1 < PER; t += 2) {
-            const unsigned a = key[t], b = key[t + 1];
-            key[t] = a > b ? a : b;
-            key[t + 1] = a > b ? b : a;
+            const Key a = key[t], b = key[t + 1];
+            const int ca = col[t], cb = col[t + 1];
+            const bool keep = a >= b;  // equal ones stay in order
+            key[t] = keep ? a : b;
+            key[t + 1] = keep ? b : a;
+            col[t] = keep ? ca : cb;
+            col[t + 1] = keep ? cb : ca;
         }
     int mine = -1;  // lane r: the r-th choice
     for (int r = 0; r < jb; ++r) {
-        const unsigned m = wave_max_u32(key[0]);
-        const int from = __ffsll((unsigned long long) __ballot(key[0] == m)) - 1;
-        if (ln == r) mine = from + WAVE * (int) (m & 15u);
+        const bool top = key[0] == wave_max_key(key[0]);
+        unsigned long long tops = __ballot(top);
+        if (tops & (tops - 1)) {
+            const int first = PQ_MAX_COLS - (int) wave_max_u32(top ? (unsigned) (PQ_MAX_COLS - col[0]) : 0u);
+            tops = __ballot(top && col[0] == first);
+        }
+        const int from = __ffsll(tops) - 1, c = __builtin_amdgcn_readlane(col[0], from);
+        if (ln == r) mine = c;
         if (ln == from) {
 #pragma unroll
-            for (int t = 0; t + 1 < PER; ++t) key[t] = key[t + 1];
-            key[PER - 1] = 0u;
+            for (int t = 0; t + 1 < PER; ++t) {
+                key[t] = key[t + 1];
+                col[t] = col[t + 1];
+            }
+            key[PER - 1] = Key(0);
         }
     }
     if (ln < PQ_NB) l.inwin[ln] = 0;
