@@ -65,17 +65,18 @@ constexpr int GJ_SC = GJ_TW * GJ_LD;  // LDS elements of one wave's tile matrix
 // Tolerances of one Jacobi.  Gram entries are scaled by a power of two so that ||J||_F^2 is about 1
 // (FP64) or 2^60 (FP32): products of two entries, and the squares of the smallest that can still ask
 // for a rotation, then neither overflow nor underflow (columns below eps ||J||_F do not take part).
+// Cosines are compared by their squares, in full precision.
 template <typename T>
 struct GramTol {
-    T tol, stop, floor2, scale;
-    __device__ __forceinline__ GramTol(T fro2, int rows, T stop_) {
+    T tol2, stop2, floor2, scale;  // squares of the two bounds on a cosine, of the smallest norm that takes part
+    __device__ __forceinline__ GramTol(T fro2, int rows, T stop) {
         int ex = 0;
         constexpr int top = sizeof(T) == 8 ? 0 : 60, lim = sizeof(T) == 8 ? 1000 : 120;
         if (fro2 > T(0) && fro2 < T(INFINITY)) ex = top - ilogb(fro2);
         ex = ex < -lim ? -lim : (ex > lim ? lim : ex);
         scale = scalbn(T(1), ex);
-        tol = sqrt(T(rows)) * Eps<T>::value;
-        stop = stop_;
+        tol2 = T(rows) * (Eps<T>::value * Eps<T>::value);
+        stop2 = stop * stop;
         floor2 = Eps<T>::value * Eps<T>::value * (fro2 * scale);
     }
 };
@@ -93,8 +94,6 @@ __device__ __forceinline__ float rsqrt_full(float x) {
     const float e = fmaf(-(x * y), y, 1.0f);
     return fmaf(y * e, fmaf(e, 0.375f, 0.5f), y);
 }
-__device__ __forceinline__ double rsqrt_estimate(double x) { return __builtin_amdgcn_rsq(x); }
-__device__ __forceinline__ float rsqrt_estimate(float x) { return __builtin_amdgcn_rsqf(x); }
 
 // Rotation (c, s) that annihilates apq for the Gram entries (app, aqq, apq) of a column pair, or
 // (1, 0) when the pair is already orthogonal to tolerance or involves a numerically zero column.
@@ -103,7 +102,7 @@ __device__ __forceinline__ float rsqrt_estimate(float x) { return __builtin_amdg
 // turn and no division.
 template <typename T>
 __device__ __forceinline__ void jacobi_rotation(T app, T aqq, T apq, const GramTol<T> &g, T &c, T &s) {
-    const bool act = app > g.floor2 && aqq > g.floor2 && fabs(apq) * rsqrt_estimate(app * aqq) > g.tol;
+    const bool act = app > g.floor2 && aqq > g.floor2 && apq * apq > g.tol2 * (app * aqq);
     const T d = aqq - app, e = T(2) * apq;
     const T r = rsqrt_full(d * d + e * e);
     const T c2 = fma(T(0.5) * fabs(d), r, T(0.5));
@@ -201,9 +200,9 @@ __device__ __forceinline__ int gram_solve(const T (&gv)[4], T *sc, bool full, co
         const T di = sc[i * (GJ_LD + 1)];
         const bool pair = full ? i < i16 : (i < GJ_B && i16 >= GJ_B);
         if (pair && di > g.floor2 && dj > g.floor2) {
-            const T cosv = fabs(gv[v] * g.scale) * rsqrt_estimate(di * dj);
-            any = any || cosv > g.tol;
-            large = large || cosv > g.stop;
+            const T x = gv[v] * g.scale, c2 = x * x, d2 = di * dj;
+            any = any || c2 > g.tol2 * d2;
+            large = large || c2 > g.stop2 * d2;
         }
     }
     if (__ballot(any) == 0) return 0;
