@@ -193,10 +193,19 @@ int tile_holders(const hcorepp_tile *t, char op, Holder<T> *h, char *hop) {
     return 2;
 }
 
-// DenseTile<T>::Gemm k / ld inference (reference src/operators/concrete/Dense.cpp:55-96, ColMajor).
+// Whether op(X) (r x c) with leading dimension ld stays inside X.
 template <typename T>
-hipError_t dense_tile_gemm(hipStream_t s, int64_t m, int64_t n, T *c, int64_t ldc, T alpha, const Holder<T> &a,
-                           char opa, const Holder<T> &b, char opb, T beta) {
+bool operand_fits(const Holder<T> &x, char op, int64_t r, int64_t c, int64_t ld) {
+    if (op == 'T') std::swap(r, c);
+    return r < 1 || c < 1 || ld * (c - 1) + r <= x.ld * (x.cols - 1) + x.rows;
+}
+
+// DenseTile<T>::Gemm k / ld inference (reference src/operators/concrete/Dense.cpp:55-96, ColMajor).  For a transposed tile
+// with fewer rows than columns the inferred ld is its columns, which reads past the tile's end: the tile's own is
+// taken there.  Operands too small for C either way are refused.
+template <typename T>
+hcorepp_status dense_tile_gemm(hipStream_t s, int64_t m, int64_t n, T *c, int64_t ldc, T alpha, const Holder<T> &a,
+                               char opa, const Holder<T> &b, char opb, T beta) {
     int64_t k = std::min(a.cols, b.rows);
     if (opa == 'T') {
         k = std::min(a.rows, b.rows);
@@ -204,10 +213,17 @@ hipError_t dense_tile_gemm(hipStream_t s, int64_t m, int64_t n, T *c, int64_t ld
     } else if (opb == 'T') {
         k = std::min(a.cols, b.cols);
     }
-    const int64_t lda = (opa == 'T') ? std::max(a.cols, k) : std::max(a.rows, m);
-    const int64_t ldb = (opb == 'T') ? std::max(b.cols, n) : std::max(b.rows, k);
-    return launch_gemm<T>(s, (int) m, (int) n, (int) k, alpha, a.data, lda, opa == 'T', b.data, ldb, opb == 'T',
-                          beta, c, ldc);
+    int64_t lda = (opa == 'T') ? std::max(a.cols, k) : std::max(a.rows, m);
+    int64_t ldb = (opb == 'T') ? std::max(b.cols, n) : std::max(b.rows, k);
+    if (!operand_fits(a, opa, m, k, lda)) lda = a.ld;
+    if (!operand_fits(b, opb, k, n, ldb)) ldb = b.ld;
+    if (m > 0 && n > 0 && (!operand_fits(a, opa, m, k, lda) || !operand_fits(b, opb, k, n, ldb)))
+        return fail(HCOREPP_ERR_INVALID, "operands %lldx%lld (%c) and %lldx%lld (%c) are too small for a %lldx%lld product",
+                    (long long) a.rows, (long long) a.cols, opa, (long long) b.rows, (long long) b.cols, opb,
+                    (long long) m, (long long) n);
+    HIP_TRY(launch_gemm<T>(s, (int) m, (int) n, (int) k, alpha, a.data, lda, opa == 'T', b.data, ldb, opb == 'T', beta, c,
+                           ldc));
+    return HCOREPP_OK;
 }
 
 // Flop model of CompressedTile<T>::Gemm, default branch (reference Compressed.cpp:335-625).
@@ -357,7 +373,7 @@ hcorepp_status gemm_plain(hcorepp_ctx *ctx, T alpha, const hcorepp_tile *A, char
         tm[ntt] = mm;
         tn[ntt] = nn;
         ntt++;
-        HIP_TRY(dense_tile_gemm<T>(s, mm, nn, t, mm, alpha_local, ad, ao, bd, bo, beta_local));
+        if ((st = dense_tile_gemm<T>(s, mm, nn, t, mm, alpha_local, ad, ao, bd, bo, beta_local))) return st;
         if (flops) *flops += 2ull * mm * nn * ad.cols;
         Holder<T> th = {mm, nn, mm, t};
         if (ntemp == 2 || (ntemp == 1 && a_idx == 0)) {
@@ -378,7 +394,7 @@ hcorepp_status gemm_plain(hcorepp_ctx *ctx, T alpha, const hcorepp_tile *A, char
         const int64_t m = tm[0], n = tn[0];
         Holder<T> cu = {C->rows, C->rank, C->rows, (T *) C->data};
         Holder<T> cv = {C->rank, C->cols, C->rank, (T *) C->data + C->rows * C->max_rank};
-        HIP_TRY(dense_tile_gemm<T>(s, m, n, W, m, beta, cu, 'N', cv, 'N', T(1)));
+        if ((st = dense_tile_gemm<T>(s, m, n, W, m, beta, cu, 'N', cv, 'N', T(1)))) return st;
         if (flops) *flops += 2ull * m * n * cu.cols;
         if (m < n)
             return fail(HCOREPP_ERR_UNSUPPORTED,
@@ -396,8 +412,8 @@ hcorepp_status gemm_plain(hcorepp_ctx *ctx, T alpha, const hcorepp_tile *A, char
 
     const Holder<T> ad = ah[a_idx], bd = bh[b_idx];
     if (C->type == HCOREPP_DENSE) {
-        HIP_TRY(dense_tile_gemm<T>(s, C->rows, C->cols, (T *) C->data, C->ld, alpha, ad, aop[a_idx], bd,
-                                   bop[b_idx], beta));
+        if ((st = dense_tile_gemm<T>(s, C->rows, C->cols, (T *) C->data, C->ld, alpha, ad, aop[a_idx], bd,
+                                   bop[b_idx], beta))) return st;
         if (flops) *flops += 2ull * C->rows * C->cols * ad.cols;
         return HCOREPP_OK;
     }
