@@ -265,9 +265,23 @@ __device__ __forceinline__ void wg_gemm_small(int M, int N, int Kd, const FA &fa
     }
 }
 
-// Whether a product of M x N output takes that form: fewer than 256 tiles of 64 x 64, one per CU.
-__host__ __device__ inline bool gemm_is_small(int64_t M, int64_t N) {
-    return ((M + GT_M - 1) / GT_M) * ((N + GT_N - 1) / GT_N) < 256;
+// Whether a product takes that form.  Its 32 x 32 tiles run in rounds of 256, one per CU, and its time grows with them; the
+// 64 x 64 form's does not while there is a tile per CU at most (225 of them: 18 us at K = 128, 74 at 960).  Times by rounds,
+// 64 x 64 form / this one:
+//   one      1.2-3.7 for every K and transpose;
+//   two      1.14-2.0 from K = 48 on, 0.95-0.99 up to 32;
+//   three    0.91 at K = 128, 0.97 at 512 and 1.1 at 8192; B transposed alone, both operands' lanes along memory, 0.91 at
+//            64, 1.01 at 128, 1.35 from 512 on; A transposed alone 0.7;
+//   four     0.56-0.84; B transposed alone 0.84 at 128, 1.07 from 512 on.
+// FP32, whose 64 x 64 form has no matrix cores: 1.1-7 for all of them.
+template <typename T>
+__host__ __device__ inline bool gemm_is_small(int64_t M, int64_t N, int64_t K, bool ta, bool tb) {
+    if (((M + GT_M - 1) / GT_M) * ((N + GT_N - 1) / GT_N) >= 256) return false;
+    const int64_t rounds = (((M + GS_T - 1) / GS_T) * ((N + GS_T - 1) / GS_T) + 255) / 256;
+    if (sizeof(T) == 4 || rounds <= 1) return true;
+    if (rounds == 2) return K > 32;
+    if (!ta && tb) return K >= (rounds == 3 ? 128 : 512);
+    return rounds == 3 && K >= 8192 && ta == tb;
 }
 
 // ---------------------------------------------------------------------------

@@ -52,7 +52,7 @@ __global__ void HCAMD_KERNEL k_y(RecompDesc<T> d) {
     ph_y<T>(d, blockIdx.x, gridDim.x, lds);
 }
 
-// The same by 32 x 32 tiles (wg_gemm_small), for a Y of fewer than 256 tiles of 64 x 64.
+// The same by 32 x 32 tiles (wg_gemm_small), where gemm_is_small says so.
 template <typename T>
 __global__ void __launch_bounds__(GS_WAVES *WAVE) k_y_small(RecompDesc<T> d, int K, int mu) {
     __shared__ T lds[GS_LDS_ELEMS];
@@ -710,7 +710,7 @@ template <typename T>
 hipError_t launch_gemm(hipStream_t s, int M, int N, int Kd, T alpha, const T *A, int64_t lda, bool ta, const T *B,
                        int64_t ldb, bool tb, T beta, T *C, int64_t ldc) {
     if (M <= 0 || N <= 0) return hipSuccess;
-    if (gemm_is_small(M, N)) {
+    if (gemm_is_small<T>(M, N, Kd, ta, tb)) {
         dim3 grid((M + GS_T - 1) / GS_T, (N + GS_T - 1) / GS_T);
         hipLaunchKernelGGL(k_gemm_small<T>, grid, dim3(GS_WAVES * WAVE), 0, s, M, N, Kd, alpha, A, lda, (int) ta, B, ldb,
                            (int) tb, beta, C, ldc);
@@ -760,7 +760,7 @@ hipError_t launch_recomp_pre(hipStream_t s, const RecompDesc<T> &d, int64_t K, i
     hipError_t e = launch_qr<T>(s, d, qu, (int) kk);
     if (e != hipSuccess) return e;
     const int ytiles = (int) (((n + GT_M - 1) / GT_M) * ((mu + GT_N - 1) / GT_N));
-    if (gemm_is_small(n, mu))
+    if (gemm_is_small<T>(n, mu, K, true, true))  // V_s and R_U^T are read as transposed operands are
         hipLaunchKernelGGL(k_y_small<T>, dim3((unsigned) ((n + GS_T - 1) / GS_T), (unsigned) ((mu + GS_T - 1) / GS_T)),
                            dim3(GS_WAVES * WAVE), 0, s, d, (int) K, (int) mu);
     else
