@@ -180,6 +180,13 @@ __global__ void HCAMD_KERNEL k_trsm_v(const CholTrsm *jobs) {
                     1.0, reinterpret_cast<double *>(smem_raw));
 }
 
+// The same with a workgroup per tile and a row per thread.
+__global__ void HCAMD_KERNEL k_trsm_v_rows(const CholTrsm *jobs) {
+    __shared__ double lds[RT_LDS];
+    const CholTrsm jb = jobs[blockIdx.x];
+    wg_rows_trsm<double>(jb.v, (int) jb.rank, (int) jb.n, jb.rank, jb.l, jb.ldl, lds);
+}
+
 // A (n x n dense) <- A - U (V V^T) U^T, with scratch W (r x r) and T (n x r); the strict upper triangle of A is
 // then set to 0, as the reference's Syrk does for a lower update.  Three launches of 32 x 32 tiles over all
 // tiles' jobs (W and A by their lower triangles): a workgroup per job, which walked its three products alone,
@@ -275,6 +282,17 @@ hipError_t launch_potrf(hipStream_t s, T *A, int n, int64_t lda, int *info) {
 template hipError_t launch_potrf<double>(hipStream_t, double *, int, int64_t, int *);
 template hipError_t launch_potrf<float>(hipStream_t, float *, int, int64_t, int *);
 hipError_t launch_trsm_v(hipStream_t s, const CholTrsm *jobs, int n, int max_rank, int len) {
+    // Workgroups of 16 vectors: the time grows with their number, at about n / 1000 us each from 500 on.  A workgroup per
+    // tile: a latency of about n us (1.3 n from 256 columns on), up to 1000 tiles of up to 256 rows at a time.  (us, 16
+    // vectors each / a tile each: 32 columns 33 / 31, with 32 vectors 120 / 50 for 2048 tiles; 64 columns 45 / 48 for 512
+    // tiles of 16 vectors, 114 / 87 for 2048; 128 columns with 64 vectors 73 / 110 for 128 tiles, 206 / 115 for 512, 742 / 241
+    // for 2048; 256 columns with 200 vectors 445 / 380 for 128, 5906 / 1858 for 2048; 512 columns with 48 722 / 1200 for 512.)
+    const int64_t groups = (max_rank + TS_NV - 1) / TS_NV;
+    const bool rows_form = len <= 32 || groups * (n < 1000 ? n : 1000) >= 10 * (int64_t) len;
+    if (n > 0 && rows_form) {
+        hipLaunchKernelGGL(k_trsm_v_rows, dim3(n), dim3(NT), 0, s, jobs);
+        return hipGetLastError();
+    }
     // jobs along y (at most 65535 per launch)
     for (int j0 = 0; j0 < n; j0 += 65535) {
         const int nj = n - j0 < 65535 ? n - j0 : 65535;

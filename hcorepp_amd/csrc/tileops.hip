@@ -67,6 +67,16 @@ __global__ void HCAMD_KERNEL k_trsm_vec(int m, int n, T alpha, const T *A, int64
                unit != 0, alpha, reinterpret_cast<T *>(smem_raw));
 }
 
+// The same with a thread per vector (thread_trsm).
+template <typename T>
+__global__ void HCAMD_KERNEL k_trsm_threads(int m, int n, T alpha, const T *A, int64_t lda, T *B, int64_t ldb, int left,
+                                            int upper, int trans, int unit) {
+    const int64_t v = (int64_t) blockIdx.x * NT + threadIdx.x;
+    if (v >= (left ? n : m)) return;
+    const bool mt = left ? trans != 0 : trans == 0;
+    thread_trsm<T>(B + (left ? v * ldb : v), left ? 1 : ldb, left ? m : n, A, lda, mt, (upper == 0) != mt, unit != 0, alpha);
+}
+
 // C's uplo triangle (diagonal included) <- alpha op(A) op(A)^T + beta C for op(A) n x k.
 template <typename T>
 __global__ void HCAMD_KERNEL k_syrk_dense(int n, int k, T alpha, const T *A, int64_t lda, int trans, T beta, T *C,
@@ -127,8 +137,12 @@ hipError_t launch_tile_trsm(hipStream_t s, int left, int upper, int trans, int u
                             const T *A, int64_t lda, T *B, int64_t ldb) {
     const int count = left ? n : m, len = left ? m : n;
     if (count <= 0 || len <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_trsm_vec<T>, dim3((count + TS_NV - 1) / TS_NV), dim3(NT), (size_t) ts_lds_bytes<T>(len), s, m,
-                       n, alpha, A, lda, B, ldb, left, upper, trans, unit);
+    if (trsm_by_thread(len, count))
+        hipLaunchKernelGGL(k_trsm_threads<T>, dim3((count + NT - 1) / NT), dim3(NT), 0, s, m, n, alpha, A, lda, B, ldb, left,
+                           upper, trans, unit);
+    else
+        hipLaunchKernelGGL(k_trsm_vec<T>, dim3((count + TS_NV - 1) / TS_NV), dim3(NT), (size_t) ts_lds_bytes<T>(len), s, m,
+                           n, alpha, A, lda, B, ldb, left, upper, trans, unit);
     return hipGetLastError();
 }
 

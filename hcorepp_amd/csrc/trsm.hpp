@@ -137,4 +137,78 @@ __device__ __forceinline__ void wg_trsm(T *X, int64_t es, int64_t vs, int nv, in
     }
 }
 
+// The same for one vector of `len` elements by one thread.
+template <typename T>
+__device__ __forceinline__ void thread_trsm(T *x, int64_t es, int len, const T *A, int64_t lda, bool mt, bool lower,
+                                            bool unit, T alpha) {
+    auto row = [&](int e) { return lower ? e : len - 1 - e; };
+    auto M = [&](int i, int j) { return mt ? A[j + i * lda] : A[i + j * lda]; };
+    for (int e = 0; e < len; ++e) {
+        const int i = row(e);
+        T s = alpha * x[i * es];
+        for (int f = 0; f < e; ++f) s -= M(i, row(f)) * x[row(f) * es];
+        x[i * es] = unit ? s : s / M(i, i);
+    }
+}
+// Whether `count` vectors of `len` elements are solved so, a thread each: where the vectors are very short, or short and so
+// many that the 1280 workgroups that fit the GPU at once take several rounds of 16 (us, 16 per workgroup / a thread each: 4
+// elements 47 / 43 at any count, 16 elements 60 / 60 at 16384 vectors, 80 / 61 at 32768, 207 / 69 at 131072; 32 elements 91 /
+// 126 at 32768, 137 / 126 at 65536, 238 / 135 at 131072).  Up to 32 elements both have the same error; beyond, a thread's
+// long sums have the larger one.
+__host__ __device__ inline bool trsm_by_thread(int64_t len, int64_t count) {
+    return len <= 8 || (len <= 32 && count >= 2048 * len);
+}
+
+// Rows of X (rows x n, column k at X + k ldx) <- X L^{-T} for lower-triangular L (n x n, ld ldl) by one workgroup, up to NT rows
+// at a time: a thread owns a row, the columns go 16 at a time, with L staged through LDS in 16 x 16 pieces.  lds:
+// RT_LDS elements.  Every thread of the workgroup must call it.
+constexpr int RT_NB = 16;
+constexpr int RT_LDS = RT_NB * (RT_NB + 1);
+template <typename T>
+__device__ __forceinline__ void wg_rows_trsm(T *X, int rows, int n, int64_t ldx, const T *L, int64_t ldl, T *lds) {
+    const int tid = (int) threadIdx.x;
+    for (int r0 = 0; r0 < rows; r0 += NT) {
+        const int a = r0 + tid;
+        const bool act = a < rows, wave = r0 + __builtin_amdgcn_readfirstlane(tid) < rows;  // this thread, this wave has rows
+        T *x = X + (act ? a : 0);
+        for (int j0 = 0; j0 < n; j0 += RT_NB) {
+            const int jb = (n - j0) < RT_NB ? (n - j0) : RT_NB;
+            T acc[RT_NB];
+#pragma unroll
+            for (int c = 0; c < RT_NB; ++c) acc[c] = (act && c < jb) ? x[(int64_t) (j0 + c) * ldx] : T(0);
+            for (int k0 = 0; k0 <= j0; k0 += RT_NB) {
+                // piece (j0, k0) of L; the last one is the diagonal block, 1 past its end
+                __syncthreads();
+                {
+                    const int c = tid % RT_NB, k = tid / RT_NB;
+                    lds[c * (RT_NB + 1) + k] = (c < jb && (k0 < j0 || k <= c)) ? L[(j0 + c) + (int64_t) (k0 + k) * ldl] : T(c == k);
+                }
+                __syncthreads();
+                if (k0 < j0 && wave) {
+                    T v[RT_NB];
+#pragma unroll
+                    for (int k = 0; k < RT_NB; ++k) v[k] = act ? x[(int64_t) (k0 + k) * ldx] : T(0);
+#pragma unroll
+                    for (int c = 0; c < RT_NB; ++c) {
+                        T p = T(0);
+#pragma unroll
+                        for (int k = 0; k < RT_NB; ++k) p = fma(v[k], lds[c * (RT_NB + 1) + k], p);
+                        acc[c] -= p;
+                    }
+                }
+            }
+            if (wave) {
+#pragma unroll
+                for (int c = 0; c < RT_NB; ++c) {
+#pragma unroll
+                    for (int k = 0; k < c; ++k) acc[c] = fma(-acc[k], lds[c * (RT_NB + 1) + k], acc[c]);
+                    acc[c] /= lds[c * (RT_NB + 1) + c];
+                    if (act && c < jb) x[(int64_t) (j0 + c) * ldx] = acc[c];
+                }
+            }
+        }
+    }
+}
+static_assert(RT_NB * RT_NB == NT, "a thread per element of a piece of L");
+
 }  // namespace hcamd
