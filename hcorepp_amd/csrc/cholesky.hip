@@ -238,6 +238,24 @@ __global__ void __launch_bounds__(GS_WAVES *WAVE) k_syrk_a(const CholSyrk *jobs)
     wg_gemm_small<double>(n, n, r, fa, fb, epi, ti, tj, lds);
 }
 
+// The same with a workgroup per tile for its three products of 64 x 64 tiles.
+__global__ void HCAMD_KERNEL k_syrk(const CholSyrk *jobs) {
+    __shared__ double lds[GT_LDS_ELEMS];
+    const CholSyrk jb = jobs[blockIdx.x];
+    const int n = (int) jb.n, r = (int) jb.rank;
+    if (r > 0) {
+        wg_gemm<double>(r, r, n, 1.0, jb.v, r, false, jb.v, r, true, 0.0, jb.w, r, lds);
+        __syncthreads();
+        wg_gemm<double>(n, r, r, 1.0, jb.u, n, false, jb.w, r, false, 0.0, jb.t, n, lds);
+        __syncthreads();
+        wg_gemm<double>(n, n, r, -1.0, jb.t, n, false, jb.u, n, true, 1.0, jb.a, jb.lda, lds);
+        __syncthreads();
+    }
+    if (n < 1) return;
+    for (ColWalk p(threadIdx.x, NT, n); p.c < n; p.next())
+        if (p.i < p.c) jb.a[p.i + (int64_t) p.c * jb.lda] = 0.0;
+}
+
 // dst (compressed, [U n x r | V r x m], max_rank cap) = src^T for src [U m x r | V r x n].
 __global__ void HCAMD_KERNEL k_transpose_factors(const CholTrans *jobs) {
     const CholTrans jb = jobs[blockIdx.x];
@@ -308,6 +326,15 @@ hipError_t set_cholesky_lds_limits() {
 hipError_t launch_syrk(hipStream_t s, const CholSyrk *jobs, int n, int max_n, int max_rank) {
     const int nn = (max_n + GS_T - 1) / GS_T, nr = (max_rank + GS_T - 1) / GS_T;
     if (nn < 1) return hipSuccess;
+    // A workgroup per tile from about one per CU on, where the three launches' tiles no longer find idle CUs (us, three
+    // launches / one workgroup per tile: 48 rows 40 / 45 for 128 tiles, 48 / 47 for 256, 68 / 57 for 512, 371 / 274 for 4000;
+    // 128 rows of rank 128 123 / 172 for 128, 407 / 289 for 512; 512 rows of rank 48 797 / 841 for 256, 1168 / 1145 for 384,
+    // 1548 / 1202 for 512).  A tile of 32 rows is one workgroup's in the three launches as well (126 / 142 for 2048).
+    const bool per_tile = max_n > 32 && n > (max_n <= 128 ? 256 : 384);
+    if (per_tile) {
+        hipLaunchKernelGGL(k_syrk, dim3(n), dim3(NT), 0, s, jobs);
+        return hipGetLastError();
+    }
     const dim3 wg(GS_WAVES * WAVE);
     // jobs along y (at most 65535 per launch)
     for (int j0 = 0; j0 < n; j0 += 65535) {
