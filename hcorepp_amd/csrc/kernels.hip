@@ -130,14 +130,17 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_qr_update(PlainQr<T> q, int j0,
     T *col = q.A + (int64_t) c * q.m + j0;
     T b[GROUPS][4];
 #pragma unroll
-    for (int t = 0; t < GROUPS; ++t) load_rows(col, 16 * (wv + WAVES * t) + 4 * k4, rows, cok, wide, b[t]);
+    for (int t = 0; t < GROUPS; ++t) {
+        load_rows<GROUPS>(col, own_rows<GROUPS>(16 * (wv + WAVES * t) + 4 * k4), rows, cok, wide, b[t]);
+        group_end<GROUPS>();
+    }
     const T *ts = q.tsave + (int64_t) (j0 / PQ_NB) * PQ_NB * PQ_NB;
     // the panel's columns hold R on and above the diagonal: unit lower in the first group of rows
     wy_block<T, WAVES, GROUPS>(
             b,
             [&](int t, T (&v)[4]) {
                 const int g = wv + WAVES * t;
-                load_rows(pcol, 16 * g + 4 * k4, rows, i16 < jb, wide, v);
+                load_rows<GROUPS>(pcol, own_rows<GROUPS>(16 * g + 4 * k4), rows, i16 < jb, wide, v);
                 if (g == 0) {
 #pragma unroll
                     for (int s = 0; s < 4; ++s) {
@@ -150,15 +153,16 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_qr_update(PlainQr<T> q, int j0,
     T nsq = T(0);
 #pragma unroll
     for (int t = 0; t < GROUPS; ++t) {
-        const int r = 16 * (wv + WAVES * t) + 4 * k4;
+        const int r = own_rows<GROUPS>(16 * (wv + WAVES * t) + 4 * k4);
         if (q.pivot) {
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                if (cok && r + s < jb) q.J[c + (int64_t) (j0 + r + s) * q.ncols] = b[t][s];
-                if (cok && r + s >= jb && r + s < rows) nsq = fma(b[t][s], b[t][s], nsq);
+                if (t == 0 && cok && r + s < jb) q.J[c + (int64_t) (j0 + r + s) * q.ncols] = b[t][s];
+                if (cok && (t > 0 || r + s >= jb) && r + s < rows) nsq = fma(b[t][s], b[t][s], nsq);
             }
         }
-        store_rows(col, r, rows, cok, wide, b[t]);
+        store_rows<GROUPS>(col, r, rows, cok, wide, b[t]);
+        group_end<GROUPS>();
     }
     if (q.pivot) {
         nsq = col_sum(nsq);
@@ -173,15 +177,17 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_qr_update(PlainQr<T> q, int j0,
     }
 }
 
-// Waves and 16-row groups per wave for a block of `rows` rows (2048 at most).  Eight waves up to 1024 rows
-// (512 threads: 256 registers hold the 1024-row blocks, which 16 waves' 128 would spill).
-template <typename F>
+// Waves and 16-row groups per wave for a block of `rows` rows (2048 at most).  Eight waves, whose 256 registers hold the
+// FP64 blocks of 1024 rows with both operands of an update and those of 2048 rows alone (sixteen waves' 128 spilled all of
+// it); FP32 blocks take half and sixteen waves beyond 1024 rows.
+template <typename T, typename F>
 static void pq_shape(int rows, F f) {
     const int g = (rows + 15) / 16;
     if (g <= 8) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
     else if (g <= 16) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 2>{});
     else if (g <= 32) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
     else if (g <= 64) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{});
+    else if constexpr (sizeof(T) == 8) f(std::integral_constant<int, 8>{}, std::integral_constant<int, 16>{});
     else f(std::integral_constant<int, 16>{}, std::integral_constant<int, 8>{});
 }
 
@@ -194,7 +200,7 @@ static hipError_t launch_qr(hipStream_t s, const RecompDesc<T> &d, const PlainQr
     }
     for (int j0 = 0; j0 < nsteps; j0 += PQ_NB) {
         const int jb = nsteps - j0 < PQ_NB ? nsteps - j0 : PQ_NB, trail = q.ncols - (j0 + jb);
-        pq_shape(q.m - j0, [&](auto waves, auto groups) {
+        pq_shape<T>(q.m - j0, [&](auto waves, auto groups) {
             constexpr int WV = decltype(waves)::value, GR = decltype(groups)::value;
             hipLaunchKernelGGL((k_qr_panel<T, WV, GR>), dim3(1), dim3(WV * WAVE), 0, s, q, d, kk, j0);
             // four columns per workgroup while that is one workgroup per CU at most: an update is bound by what one CU
@@ -496,13 +502,16 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_recon(RecompDesc<T> d) {
     const T sg = cok ? w.sig[j] : T(0);
     T b[GROUPS][4];
 #pragma unroll
-    for (int t = 0; t < GROUPS; ++t)
+    for (int t = 0; t < GROUPS; ++t) {
+        const int r0 = own_rows<GROUPS>(16 * (wv + WAVES * t) + 4 * k4);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const int row = 16 * (wv + WAVES * t) + 4 * k4 + s;
+            const int row = r0 + s;
             const T v = (cok && row < filled) ? src[row + (int64_t) j * filled] : T(0);
             b[t][s] = side ? v * sg : (sg > T(0) ? v / sg : T(0));
         }
+        group_end<GROUPS>();
+    }
     const T *A = side ? w.y : w.us, *tsave = side ? w.t_y : w.t_u;  // ld rows
     // [v1 sigma; 0] vanishes below row kt, where reflectors kt.. of Q_Y act as the identity (each is zero
     // above its own row), so only the first kt are applied
@@ -519,7 +528,7 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_recon(RecompDesc<T> d) {
                 b,
                 [&](int t, T (&v)[4]) {
                     const int g = wv + WAVES * t;
-                    load_rows(pcol, 16 * g + 4 * k4, rows, i16 < jb && g >= p, wide, v);
+                    load_rows<GROUPS>(pcol, own_rows<GROUPS>(16 * g + 4 * k4), rows, i16 < jb && g >= p, wide, v);
                     if (g == p) {
 #pragma unroll
                         for (int s = 0; s < 4; ++s) {
@@ -533,15 +542,18 @@ __global__ void __launch_bounds__(WAVES *WAVE) k_recon(RecompDesc<T> d) {
     if (c >= r) return;
     T *cu = d.cdata, *cv = d.cdata + (int64_t) d.m * d.max_rank;
 #pragma unroll
-    for (int t = 0; t < GROUPS; ++t)
+    for (int t = 0; t < GROUPS; ++t) {
+        const int r0 = own_rows<GROUPS>(16 * (wv + WAVES * t) + 4 * k4);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const int row = 16 * (wv + WAVES * t) + 4 * k4 + s;
+            const int row = r0 + s;
             if (row < rows) {
                 if (side) cv[c + (int64_t) row * r] = b[t][s];
                 else cu[row + (int64_t) c * d.m] = b[t][s];
             }
         }
+        group_end<GROUPS>();
+    }
 }
 
 __global__ void k_set_i64(int64_t *p, int64_t v) {
@@ -772,7 +784,7 @@ hipError_t launch_recomp_pre(hipStream_t s, const RecompDesc<T> &d, int64_t K, i
 
 template <typename T>
 hipError_t launch_recomp_post(hipStream_t s, const RecompDesc<T> &d, int64_t r) {
-    pq_shape(d.m > d.n ? d.m : d.n, [&](auto waves, auto groups) {
+    pq_shape<T>(d.m > d.n ? d.m : d.n, [&](auto waves, auto groups) {
         constexpr int WV = decltype(waves)::value, GR = decltype(groups)::value;
         hipLaunchKernelGGL((k_recon<T, WV, GR>), dim3((unsigned) ((r + PQ_NB - 1) / PQ_NB), 2), dim3(WV * WAVE), 0, s, d);
     });

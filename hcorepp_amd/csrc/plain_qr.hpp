@@ -101,19 +101,27 @@ __device__ __forceinline__ void store4(float *q, bool wide, const float (&v)[4])
     if (wide) *reinterpret_cast<float4 *>(q) = float4{v[0], v[1], v[2], v[3]};
     else q[0] = v[0], q[1] = v[1], q[2] = v[2], q[3] = v[3];
 }
-// The same for rows r .. r + 3 of a column of `rows` rows, zero (not written) past its end.
-template <typename T>
+// Rows r .. r + 3 of a column of `rows` rows, zero (not written) past its end.  Blocks of more than eight groups make every
+// load, at the column's last row where its own is past the end: with branches around them the branches' state took the
+// registers.  (The kernels of 1025 to 2048 rows had 310 to 750 bytes of scratch per lane; below about 270 each launch is 60 us
+// shorter, an update of rank 1 in a 2048 x 2048 tile 260 -> 170 us, of rank 128 6.66 -> 3.28 ms.)
+template <int GROUPS, typename T>
 __device__ __forceinline__ void load_rows(const T *col, int r, int rows, bool ok, bool wide, T (&v)[4]) {
-    if (ok && r + 3 < rows) {
+    if constexpr (GROUPS > 8) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) v[s] = col[r + s < rows ? r + s : rows - 1];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) v[s] = (ok && r + s < rows) ? v[s] : T(0);
+    } else if (ok && r + 3 < rows) {
         load4(col + r, wide, v);
     } else {
 #pragma unroll
         for (int s = 0; s < 4; ++s) v[s] = (ok && r + s < rows) ? col[r + s] : T(0);
     }
 }
-template <typename T>
+template <int GROUPS, typename T>
 __device__ __forceinline__ void store_rows(T *col, int r, int rows, bool ok, bool wide, const T (&v)[4]) {
-    if (ok && r + 3 < rows) {
+    if (GROUPS <= 8 && ok && r + 3 < rows) {
         store4(col + r, wide, v);
     } else {
 #pragma unroll
@@ -125,6 +133,22 @@ __device__ __forceinline__ void store_rows(T *col, int r, int rows, bool ok, boo
 template <typename T>
 __device__ __forceinline__ bool wide_columns(const T *A, int64_t ld) {
     return (reinterpret_cast<uintptr_t>(A) & 15) == 0 && (ld * (int64_t) sizeof(T)) % 16 == 0;
+}
+
+// Blocks of more than eight groups leave no registers for the next groups' addresses and operands, nor for row numbers
+// kept from the loads to the stores: group_end keeps a group's instructions together, own_rows gives row numbers that are
+// computed anew.
+template <int GROUPS>
+__device__ __forceinline__ void group_end() {
+    if constexpr (GROUPS > 8) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+template <int GROUPS>
+__device__ __forceinline__ int own_rows(int r) {
+    if constexpr (GROUPS > 8) asm volatile("" : "+v"(r));
+    return r;
 }
 
 __device__ __forceinline__ double rcp_full(double d) {
@@ -194,28 +218,43 @@ struct PanelLds {
 template <typename T, int WAVES, int GROUPS>
 __device__ __forceinline__ T panel_factor(T (&p)[GROUPS][4], int jb, T *tau, PanelLds<T, WAVES> &l) {
     const int ln = lane_id(), i16 = ln & 15, k4 = ln >> 4, wv = wave_id();
-    T xs[GROUPS][4];  // the current column, rows below its pivot (0 elsewhere)
+    // the current column, rows below its pivot (0 elsewhere): kept from its products to the update after them where
+    // the registers hold it beside p, broadcast twice in blocks of more than eight groups
+    constexpr bool KEEP = GROUPS <= 8;
+    T xs[KEEP ? GROUPS : 1][4];
     T myscal = T(0);
     int c = i16;      // this lane's column
-    // the products with column nj, which is in lane 0 of each row of lanes
+    // column nj, which is in lane 0 of each row of lanes
+    auto current = [&](int t, int s, int nj) {
+        const T x = row_move<DPP_ROW_BCAST0>(p[t][s]);
+        return (t == 0 && wv == 0 && 4 * k4 + s <= nj) ? T(0) : x;
+    };
+    // the products with it
     auto products = [&](int nj, int buf) {
+        if constexpr (KEEP) {
 #pragma unroll
-        for (int t = 0; t < GROUPS; ++t)
+            for (int t = 0; t < GROUPS; ++t)
 #pragma unroll
-            for (int s = 0; s < 4; ++s) xs[t][s] = row_move<DPP_ROW_BCAST0>(p[t][s]);
+                for (int s = 0; s < 4; ++s) xs[t][s] = row_move<DPP_ROW_BCAST0>(p[t][s]);
+        }
         if (wv == 0) {
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const int r = 4 * k4 + s;
                 if (r == nj) l.xrow[buf][c] = p[0][s];
-                if (r <= nj) xs[0][s] = T(0);
+                if (KEEP && r <= nj) xs[0][s] = T(0);
             }
         }
         T acc[4] = {T(0), T(0), T(0), T(0)};
 #pragma unroll
-        for (int t = 0; t < GROUPS; ++t)
+        for (int t = 0; t < GROUPS; ++t) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) acc[s] = fma(xs[t][s], p[t][s], acc[s]);
+            for (int s = 0; s < 4; ++s) {
+                if constexpr (KEEP) acc[s] = fma(xs[t][s], p[t][s], acc[s]);
+                else acc[s] = fma(current(t, s, nj), p[t][s], acc[s]);
+            }
+            group_end<GROUPS>();
+        }
         const T sum = col_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
         if (k4 == 0) l.red[buf][wv][c] = sum;
     };
@@ -239,9 +278,14 @@ __device__ __forceinline__ T panel_factor(T (&p)[GROUPS][4], int jb, T *tau, Pan
         const T gk = (c > jj && c < jb) ? tj * wk : T(0);
         const T gp = gk * scal;
 #pragma unroll
-        for (int t = 0; t < GROUPS; ++t)
+        for (int t = 0; t < GROUPS; ++t) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) p[t][q] = fma(-gp, xs[t][q], p[t][q]);
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (KEEP) p[t][q] = fma(-gp, xs[t][q], p[t][q]);
+                else p[t][q] = fma(-gp, current(t, q, jj), p[t][q]);
+            }
+            group_end<GROUPS>();
+        }
         if (wv == 0) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -408,21 +452,25 @@ __device__ __forceinline__ void wg_panel(const PlainQr<T> &q, int j0, PanelLds<T
     T p[GROUPS][4];
     const T *src = column(i16 < jb ? i16 : 0);
 #pragma unroll
-    for (int t = 0; t < GROUPS; ++t) load_rows(src, 16 * (wv + WAVES * t) + 4 * k4, rows, i16 < jb, wide, p[t]);
+    for (int t = 0; t < GROUPS; ++t) {
+        load_rows<GROUPS>(src, own_rows<GROUPS>(16 * (wv + WAVES * t) + 4 * k4), rows, i16 < jb, wide, p[t]);
+        group_end<GROUPS>();
+    }
     const T scal = panel_factor<T, WAVES, GROUPS>(p, jb, q.tau + j0, l);
     const int c = (i16 + jb) & 15;
     T *dst = column(c < jb ? c : 0);
 #pragma unroll
     for (int t = 0; t < GROUPS; ++t) {
-        const int r = 16 * (wv + WAVES * t) + 4 * k4;
+        const int r = own_rows<GROUPS>(16 * (wv + WAVES * t) + 4 * k4);
         T v[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            v[s] = r + s > c ? scal * p[t][s] : p[t][s];
+            v[s] = (t > 0 || r + s > c) ? scal * p[t][s] : p[t][s];
             // R[j0 + r, j0 + c] for the core
-            if (q.pivot && c < jb && r + s <= c) q.J[l.piv[c] + (int64_t) (j0 + r + s) * q.ncols] = p[t][s];
+            if (t == 0 && q.pivot && c < jb && r + s <= c) q.J[l.piv[c] + (int64_t) (j0 + r + s) * q.ncols] = p[t][s];
         }
-        store_rows(dst, r, rows, c < jb, wide, v);
+        store_rows<GROUPS>(dst, r, rows, c < jb, wide, v);
+        group_end<GROUPS>();
     }
     T *ts = q.tsave + (int64_t) (j0 / PQ_NB) * PQ_NB * PQ_NB;
     for (int e = threadIdx.x; e < PQ_NB * PQ_NB; e += WAVES * WAVE) ts[e] = l.t[e % PQ_NB][e / PQ_NB];
@@ -445,16 +493,20 @@ __device__ __forceinline__ int pq_prow(int i) {
 // b <- (I - P op(T) P^T) b for a register block b, on the matrix cores; op(T) is T^T with `trans`.  pa(t, v) gives
 // P, zero outside its rows: rows 16 G + 4 k4 .. + 3 of column i16, G = wave + WAVES t; groups below g0 are zero in P
 // and skipped.  tm(i, j) gives T.  Two barriers; every wave of the workgroup calls it.  The second product takes P
-// with its rows along the lanes, which each wave gets from its own LDS: reading both forms from memory, a CU moved
-// P twice (update of 1024 rows 19.0 us, 17.9 now; reconstruction of 1024 rows and rank 341 435 us, 365 now).
+// with its rows along the lanes, which each wave gets from its own LDS: reading both forms from memory, a CU moved P
+// twice (update of 1024 rows 19.0 us, 17.9 now; reconstruction of 1024 rows and rank 341 435 us, 365 now).  Blocks of more
+// than four groups turn a group as it is needed, blocks of more than eight read P again, for the registers.
 template <typename T, int WAVES, int GROUPS, typename PA, typename TM>
 __device__ __forceinline__ void wy_block(T (&b)[GROUPS][4], const PA &pa, const TM &tm, bool trans, int g0,
                                          WyLds<T, WAVES> &l) {
     using MF = Mfma16<T>;
+    constexpr bool KEEP = GROUPS <= 8, EARLY = GROUPS <= 4;
     const int ln = lane_id(), i16 = ln & 15, k4 = ln >> 4, wv = wave_id();
-    T a[GROUPS][4], c[GROUPS][4], top[4];
+    T a[KEEP ? GROUPS : 1][4], c[EARLY ? GROUPS : 1][4], top[4];
+    if constexpr (KEEP) {
 #pragma unroll
-    for (int t = 0; t < GROUPS; ++t) pa(t, a[t]);
+        for (int t = 0; t < GROUPS; ++t) pa(t, a[t]);
+    }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
         const int k = MF::row(s, k4);
@@ -462,22 +514,27 @@ __device__ __forceinline__ void wy_block(T (&b)[GROUPS][4], const PA &pa, const 
     }
     T *tile = l.part[wv];
     const int pr = pq_prow<T>(i16);
+    auto turn = [&](const T (&x)[4], T (&y)[4]) {
 #pragma unroll
-    for (int t = 0; t < GROUPS; ++t) {
-        if (wv + WAVES * t < g0) continue;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) tile[i16 * (PQ_NB + 1) + 4 * k4 + s] = a[t][s];
+        for (int s = 0; s < 4; ++s) tile[i16 * (PQ_NB + 1) + 4 * k4 + s] = x[s];
         wave_fence();
 #pragma unroll
-        for (int s = 0; s < 4; ++s) c[t][s] = tile[MF::row(s, k4) * (PQ_NB + 1) + pr];
+        for (int s = 0; s < 4; ++s) y[s] = tile[MF::row(s, k4) * (PQ_NB + 1) + pr];
         wave_fence();
+    };
+    if constexpr (EARLY) {
+#pragma unroll
+        for (int t = 0; t < GROUPS; ++t)
+            if (wv + WAVES * t >= g0) turn(a[t], c[t]);
     }
     typename MF::acc acc = MF::zero();
 #pragma unroll
     for (int t = 0; t < GROUPS; ++t) {
         if (wv + WAVES * t < g0) continue;
+        if constexpr (!KEEP) pa(t, a[0]);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) acc = MF::mma(a[t][s], b[t][s], acc);
+        for (int s = 0; s < 4; ++s) acc = MF::mma(a[KEEP ? t : 0][s], b[t][s], acc);
+        group_end<GROUPS>();
     }
 #pragma unroll
     for (int v = 0; v < 4; ++v) l.part[wv][MF::row(v, k4) * PQ_NB + i16] = acc[v];
@@ -495,11 +552,14 @@ __device__ __forceinline__ void wy_block(T (&b)[GROUPS][4], const PA &pa, const 
 #pragma unroll
     for (int t = 0; t < GROUPS; ++t) {
         if (wv + WAVES * t < g0) continue;
+        if constexpr (!KEEP) pa(t, a[0]);
+        if constexpr (!EARLY) turn(a[KEEP ? t : 0], c[0]);
         typename MF::acc d = MF::zero();
 #pragma unroll
-        for (int s = 0; s < 4; ++s) d = MF::mma(c[t][s], wp[s], d);
+        for (int s = 0; s < 4; ++s) d = MF::mma(c[EARLY ? t : 0][s], wp[s], d);
 #pragma unroll
         for (int v = 0; v < 4; ++v) b[t][v] -= d[v];
+        group_end<GROUPS>();
     }
 }
 
