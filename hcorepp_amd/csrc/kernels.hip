@@ -68,7 +68,7 @@ __global__ void __launch_bounds__(GS_WAVES *WAVE) k_y_small(RecompDesc<T> d, int
 
 // ---------------------------------------------------------------------------
 // Blocked QR of the plain form (plain_qr.hpp): one launch factors a panel (one workgroup, window pivoting
-// included for the QR of Y); the next applies its block reflector to the trailing columns, 16 columns
+// included for the QR of Y); the next applies its block reflector to the trailing columns, 4 or 16 columns
 // per workgroup over the whole GPU.  The operand's pointers and sizes come as arguments: the host knows
 // them, and a read of the workspace header at the start of every launch took 2 us.
 // ---------------------------------------------------------------------------
@@ -205,7 +205,9 @@ static hipError_t launch_qr(hipStream_t s, const RecompDesc<T> &d, const PlainQr
             hipLaunchKernelGGL((k_qr_panel<T, WV, GR>), dim3(1), dim3(WV * WAVE), 0, s, q, d, kk, j0);
             // four columns per workgroup while that is one workgroup per CU at most: an update is bound by what one CU
             // moves of its columns, not by the matrix cores, which 16 would fill (1024 rows 24.8 us with 16, 20.9 with
-            // 8, 19.0 with 4; 512 rows 13.8, 11.9, 11.0; 256 rows 8.4, 7.6, 7.1; 17.9, 10.5 and 7.0 since P is read once)
+            // 8, 19.0 with 4; 512 rows 13.8, 11.9, 11.0; 256 rows 8.4, 7.6, 7.1; 17.9, 10.5 and 7.0 since P is read once).
+            // Beyond, either is within 1 % of the whole update: 600 rows, 1200 stacked columns 10.61 ms with 16, 10.68 with 4,
+            // 700 rows and 1400 columns 14.07 and 14.19
             const int uc = trail <= 4 * 256 ? 4 : PQ_NB;
             if (trail > 0)
                 hipLaunchKernelGGL((k_qr_update<T, WV, GR>), dim3((trail + uc - 1) / uc), dim3(WV * WAVE), 0, s, q, j0, uc);

@@ -65,6 +65,10 @@ hipError_t launch_gemm(hipStream_t s, int M, int N, int Kd, T alpha, const T *A,
 // (column norms).  m, n <= 2048.
 // The records of the multi-workgroup Jacobi (at most 32 elements per column and 1 K) fit the workspace
 // region they use, (kk + 17) kk elements, from 48 columns on.
+// Where the line lies: us of a whole update of 256 rows, one workgroup / many, for cores that keep all their columns and for
+// cores cut to a part of them, which pay 10 to 20 us for reading the width: 72 columns 751 / 721 and 649 / 712, 88 1204 / 925
+// and 995 / 1006, 104 1493 / 1097 and 1256 / 1276, 112 1559 / 1113 and 1485 / 1491, 128 1892 / 1250 and 1455 / 1468.  Most cores
+// are cut; from 112 on, what they lose is below 1 % of their update.
 constexpr int MW_MIN_COLS = 112;
 template <typename T>
 hipError_t launch_recomp_pre(hipStream_t s, const RecompDesc<T> &d, int64_t K, int32_t *jflags, int64_t *host, T *cn);

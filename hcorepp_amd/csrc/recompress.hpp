@@ -1293,7 +1293,7 @@ __device__ void ph_svd_finish(const RecompDesc<T> &d, int sweeps) {
 // The core moves into the kernel's dynamic LDS for the whole iteration where it fits with the waves'
 // tile matrices (up to 93 square columns), so that its sweeps read no global memory; wider cores pass
 // through it by super-blocks (wg_staged_jacobi), the waves sharing tiles where the LDS holds fewer
-// than four at a time (32 columns per super-block up to 138 rows, 16 up to 276, 8 up to 554); taller
+// than four at a time (32 columns per super-block up to 137 rows, 16 up to 277, 8 up to 555); taller
 // ones are rotated in global memory.
 // ---------------------------------------------------------------------------
 constexpr int64_t BATCH_LDS_BYTES = 78 * 1024;  // dynamic LDS per workgroup of the batched kernel
