@@ -433,7 +433,8 @@ hcorepp_status recompress_plain(hcorepp_ctx *ctx, T alpha, const Holder<T> &ad, 
     if (ad.rows != m || bd.cols != n || bd.rows != arank)
         return fail(HCOREPP_ERR_INVALID, "operand shapes do not match C (%lldx%lld)", (long long) m,
                     (long long) n);
-    if (std::max(m, n) > 2048) return fail(HCOREPP_ERR_UNSUPPORTED, "tile too tall for the LDS panel (rows %lld)", (long long) m);
+    if (std::max(m, n) > 2048)
+        return fail(HCOREPP_ERR_UNSUPPORTED, "a QR of %lld rows exceeds the limit of 2048", (long long) std::max(m, n));
     if (std::min(m, K) > JACOBI_ROWS_MAX)
         return fail(HCOREPP_ERR_UNSUPPORTED, "stacked rank %lld exceeds the core SVD limit %d", (long long) K,
                     JACOBI_ROWS_MAX);

@@ -28,3 +28,14 @@ def test_tall_blocks(ctx, m, n, ra, rc, dtype, eps):
     assert rel_fro(C.to_dense(), full) < 100 * (ra + rc + 1) * eps
     u = C.factors()[0].astype(np.float64)
     assert np.abs(u.T @ u - np.eye(u.shape[1])).max() < 100 * (ra + rc + 1) * eps
+
+
+@pytest.mark.parametrize("m,n", [(10, 2049), (2050, 10)])
+def test_taller_blocks_are_refused(ctx, m, n):
+    """More than 2048 rows of either QR, with the number and the limit in the message; C stays as it was."""
+    import hcorepp_amd as H
+    a, b, c = (np.ones((m, 1)), np.ones((1, 9))), (np.ones((9, 1)), np.ones((1, n))), (np.ones((m, 1)), np.ones((1, n)))
+    C = H.CompressedTile(*c, max_rank=2)
+    with pytest.raises(H.HCoreError, match=f"UNSUPPORTED.*{max(m, n)} rows.*2048"):
+        H.HCore.gemm(1.0, H.CompressedTile(*a), H.CompressedTile(*b), 1.0, C, ctx, H.CompressionParameters(1e-8))
+    assert C.rank == 1 and all(np.array_equal(x, y) for x, y in zip(C.factors(), c))
