@@ -80,39 +80,6 @@ __device__ __forceinline__ T wg_sum(T v, T *red) {
     return s;
 }
 
-// Reduce NV independent partial sums held by every lane of a wave so that,
-// on return, every lane holds the full wave sum of one value index:
-// index = lane >> (6 - log2 NV) (lane bit 5 is the index MSB).  Each halving
-// round exchanges half of the live values with the partner lane, so the total
-// cost is NV - 1 + (6 - log2 NV) shuffles instead of 6 * NV.  Written with
-// compile-time recursion so that the value array stays in registers.
-template <typename T, int NV, int CNT, int OFF>
-struct MultiSum {
-    static __device__ __forceinline__ void run(T (&v)[NV], int l) {
-        if constexpr (CNT > 1) {
-            constexpr int HALF = CNT / 2;
-            const bool upper = (l & OFF) != 0;
-#pragma unroll
-            for (int i = 0; i < HALF; ++i) {
-                const T send = upper ? v[i] : v[i + HALF];
-                const T keep = upper ? v[i + HALF] : v[i];
-                v[i] = keep + __shfl_xor(send, OFF, WAVE);
-            }
-            MultiSum<T, NV, HALF, OFF / 2>::run(v, l);
-        } else if constexpr (OFF >= 1) {
-            v[0] += __shfl_xor(v[0], OFF, WAVE);
-            MultiSum<T, NV, 1, OFF / 2>::run(v, l);
-        }
-    }
-};
-
-template <typename T, int NV>
-__device__ __forceinline__ T wave_multi_sum(T (&v)[NV]) {
-    static_assert((NV & (NV - 1)) == 0 && NV <= 64, "NV must be a power of two <= 64");
-    MultiSum<T, NV, NV, 32>::run(v, lane_id());
-    return v[0];
-}
-
 // ---------------------------------------------------------------------------
 // Cross-lane exchanges on 32- or 64-bit values without the LDS crossbar: DPP row
 // permutations (row_mirror, row_half_mirror, quad_perm) and gfx950's permlane swaps.
@@ -227,8 +194,9 @@ struct MultiSumFast {
     }
 };
 
-// Same result convention as wave_multi_sum (lane l holds the total of value index
-// l >> (6 - log2 NV)), computed with permlane swaps and DPP instead of ds_bpermute.
+// The wave's sums of NV values per lane: lane l returns the total of value index l >> (6 - log2 NV) (lane bit 5 is
+// the index's highest).  Each level exchanges half of the values that are left with the partner lane, so NV - 1 + (6 - log2 NV)
+// exchanges do where 6 NV would for one value after the other; compile-time recursion keeps the values in registers.
 template <typename T, int NV>
 __device__ __forceinline__ T wave_multi_sum_fast(T (&v)[NV]) {
     static_assert((NV & (NV - 1)) == 0 && NV <= 64, "NV must be a power of two <= 64");
@@ -257,13 +225,13 @@ __host__ __device__ __forceinline__ constexpr int log2_const() {
     return NV <= 1 ? 0 : 1 + log2_const<NV / 2>();
 }
 
-// Value index held by lane l after wave_multi_sum<NV>.
+// Value index held by lane l after wave_multi_sum_fast<NV>.
 template <int NV>
 __device__ __forceinline__ int wave_multi_sum_index(int l) {
     return l >> (6 - log2_const<NV>());
 }
 
-// Lane that holds value index j after wave_multi_sum<NV>: index bits map to lane bits 5..(6-log2 NV).
+// Lane that holds value index j after wave_multi_sum_fast<NV>: index bits map to lane bits 5..(6-log2 NV).
 template <int NV>
 __device__ __forceinline__ constexpr int multi_sum_src_lane(int j) {
     return j << (6 - log2_const<NV>());
@@ -313,20 +281,6 @@ __device__ __forceinline__ double lane_fetch(double v, int src) {
 __device__ __forceinline__ void wave_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-}
-
-// dst[e] = src[e] for e in [0, n) by the whole workgroup, four loads in flight per thread.
-template <typename T>
-__device__ __forceinline__ void wg_copy(T *dst, const T *src, int64_t n) {
-    int64_t e = threadIdx.x;
-    for (; e + 3 * NT < n; e += 4 * NT) {
-        const T a = src[e], b = src[e + NT], c = src[e + 2 * NT], d = src[e + 3 * NT];
-        dst[e] = a;
-        dst[e + NT] = b;
-        dst[e + 2 * NT] = c;
-        dst[e + 3 * NT] = d;
-    }
-    for (; e < n; e += NT) dst[e] = src[e];
 }
 
 template <typename T>

@@ -164,19 +164,14 @@ __device__ __forceinline__ void wg_gemm_tile_core(int M, int N, int Kd, const FA
 
 template <typename T>
 __device__ void wg_gemm_tile(int M, int N, int Kd, T alpha, const T *A, int64_t lda, bool ta, const T *B,
-                             int64_t ldb, bool tb, T beta, T *C, int64_t ldc, int ti, int tj, T *lds,
-                             bool upper_b = false) {
+                             int64_t ldb, bool tb, T beta, T *C, int64_t ldc, int ti, int tj, T *lds) {
     auto fa = [=](int i, int k) -> T { return ta ? A[k + (int64_t) i * lda] : A[i + (int64_t) k * lda]; };
-    auto fb = [=](int k, int j) -> T {
-        if (upper_b && k < j) return T(0);
-        return tb ? B[j + (int64_t) k * ldb] : B[k + (int64_t) j * ldb];
-    };
+    auto fb = [=](int k, int j) -> T { return tb ? B[j + (int64_t) k * ldb] : B[k + (int64_t) j * ldb]; };
     auto epi = [=](int gi, int gj, T v) {
         T *c = C + gi + (int64_t) gj * ldc;
         *c = (beta == T(0)) ? alpha * v : alpha * v + beta * *c;
     };
-    // with upper_b, op(B)(k, j) vanishes for k < j: the tile's columns start at tj * GT_N
-    wg_gemm_tile_core<T>(M, N, Kd, fa, fb, !ta, tb, epi, ti, tj, lds, upper_b ? tj * GT_N : 0);
+    wg_gemm_tile_core<T>(M, N, Kd, fa, fb, !ta, tb, epi, ti, tj, lds);
 }
 
 // One 64 x 64 tile of C (M x N, ld ldc) = sum_k fa(i, k) fb(k, j) for operands given as element
@@ -190,7 +185,6 @@ __device__ void wg_gemm_tile_fn(int M, int N, int Kd, const FA &fa, const FB &fb
 }
 
 // Whole-matrix GEMM by one workgroup (loops over all 64x64 tiles).
-// `upper_b` treats op(B)(k, j) as zero for k < j (a transposed upper-triangular factor).
 template <typename T>
 __device__ void wg_gemm(int M, int N, int Kd, T alpha, const T *A, int64_t lda, bool ta, const T *B, int64_t ldb,
                         bool tb, T beta, T *C, int64_t ldc, T *lds) {

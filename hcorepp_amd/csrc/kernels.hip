@@ -282,10 +282,6 @@ __global__ void __launch_bounds__(JW_THREADS) k_jacobi_wg(RecompDesc<T> d) {
     Ws<T> w = ws_of(d);
     const Dims z = dims_of(d, w);
     const int rows = z.mu, nc = z.kt, ldj = rows | 1, ldv = nc | 1;
-    if (rows > JACOBI_ROWS_MAX) {
-        if (threadIdx.x == 0) w.hdr[HDR_STATUS] |= STATUS_TOO_BIG;
-        return;
-    }
     const T fro2 = (T) __longlong_as_double(w.hdr[HDR_JFRO2]), stop = JacobiStopCos<T>::tight;
     T *Jl = lds + gram_jacobi_lds<T>(NW), *Vl = Jl + (int64_t) ldj * nc;
     const bool jin = (int64_t) ldj * nc <= cap, vin = (int64_t) (ldj + ldv) * nc <= cap;
@@ -658,7 +654,7 @@ __global__ void HCAMD_KERNEL k_batched(const BatchEntry<T> *entries, const int32
         if (z.K <= d.kmax && (d.rank_model || !(d.model_tol > 0.0))) ph_features<T>(d, lds);
         uint64_t t_qru = 0, t_y = 0, t_qry = 0, t_svd = 0, t_ru = 0;
         if (z.K <= d.kmax) {
-            wg_geqrf<T, PB>(d.m, z.K, w.us, d.m, w.tau_u, w.t_u, lds, nullptr, w.hdr, u_in_place, stacked_u(d, z.K));
+            wg_geqrf<T, PB>(d.m, z.K, w.us, d.m, w.tau_u, w.t_u, lds, w.hdr, u_in_place, stacked_u(d, z.K));
             __syncthreads();
             t_qru = HCAMD_TSTAMP();
             ph_y<T>(d, 0, 1, lds);
@@ -835,12 +831,14 @@ hipError_t launch_batched(hipStream_t s, const BatchEntry<T> *entries, const int
 template <typename T>
 hipError_t set_kernel_lds_limits(int64_t lds_bytes) {
     // Allow the dynamic-LDS kernels to use more than the default 64 KB.
-    const void *fns[] = {
-            (const void *) k_batched<T, 16>, (const void *) k_batched<T, 8>, (const void *) k_batched<T, 4>,
-    };
-    for (const void *f : fns) {
-        hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds_bytes);
-        if (e != hipSuccess) return e;
+    if constexpr (sizeof(T) == 8) {  // the batched form is FP64
+        const void *fns[] = {
+                (const void *) k_batched<T, 16>, (const void *) k_batched<T, 8>, (const void *) k_batched<T, 4>,
+        };
+        for (const void *f : fns) {
+            hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds_bytes);
+            if (e != hipSuccess) return e;
+        }
     }
     return hipFuncSetAttribute((const void *) k_jacobi_wg<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int) JW_LDS_BYTES);
@@ -854,11 +852,11 @@ hipError_t set_kernel_lds_limits(int64_t lds_bytes) {
     template hipError_t launch_recomp_post<T>(hipStream_t, const RecompDesc<T> &, int64_t);                      \
     template hipError_t launch_readjust_ddc<T>(hipStream_t, const T *, int64_t, int64_t, T *);                   \
     template hipError_t launch_fill_identity<T>(hipStream_t, T *, int64_t);                                      \
-    template hipError_t launch_batched<T>(hipStream_t, const BatchEntry<T> *, const int32_t *, int64_t,          \
-                                          BatchCounters *, int, int64_t, int, int, char *, int64_t, int64_t *);  \
     template hipError_t set_kernel_lds_limits<T>(int64_t);
 
 HCAMD_INSTANTIATE(double)
 HCAMD_INSTANTIATE(float)
+template hipError_t launch_batched<double>(hipStream_t, const BatchEntry<double> *, const int32_t *, int64_t,
+                                           BatchCounters *, int, int64_t, int, int, char *, int64_t, int64_t *);
 
 }  // namespace hcamd

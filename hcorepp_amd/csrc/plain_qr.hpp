@@ -195,8 +195,7 @@ struct PanelLds {
     T t[PQ_NB][PQ_NB + 1];        // products of the reflectors, then the T factor
     T tau[PQ_NB];
     int piv[PQ_MAX_COLS];         // window pivoting: the trailing columns by position
-    int sel[PQ_NB];               // the positions chosen,
-    int vac[PQ_NB], disp[PQ_NB];  // those beyond the panel, and the panel's positions that were not
+    int vac[PQ_NB], disp[PQ_NB];  // chosen positions beyond the panel, and the panel's positions that were not chosen
     int inwin[PQ_NB];
     int stop;
 };

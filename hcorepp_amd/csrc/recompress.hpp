@@ -20,9 +20,9 @@
 // (R_U R_V^T)^T, a triangular preconditioner that cuts the Jacobi sweep count ~3x.
 // "V carries Sigma" (:597-599) is the V1 Sigma factor.
 //
-// Every phase is executed by a whole workgroup of NT threads; the same code
-// runs one phase per launch (plain path) or all phases in one persistent
-// launch (batched path).
+// Every phase is executed by a whole workgroup of NT threads, all of them in one persistent launch (batched
+// form).  The plain form, whose launches spread one update over the GPU, takes the workspace, the stacking, the
+// product Y and the rank rule from here; its other kernels are in kernels.hip and plain_qr.hpp.
 #pragma once
 
 #include "device_common.hpp"
@@ -764,17 +764,14 @@ __host__ __device__ inline bool window_pivot_fits(int64_t m, int64_t ncols, int 
 // ---------------------------------------------------------------------------
 // Blocked Householder QR (LAPACK dgeqrf convention) of A (m x ncols, ld lda) in
 // place; tau[0..min(m,ncols)); the T factor of panel p is saved to tsave[p*PB*PB].
-// With piv non-null, each panel starts with window pivoting (window_pivot) and
-// piv[0..ncols) receives the column permutation: A P = Q R.
 // ---------------------------------------------------------------------------
 
-// One panel of the blocked QR below: window pivoting (when piv is given), Householder
-// factorisation of columns [j0, j0 + jb) over rows [j0, m), write-back, and the compact-WY T
+// One panel of the blocked QR below: Householder factorisation of columns [j0, j0 + jb) over rows [j0, m), write-back, and the compact-WY T
 // (saved to tsave[j0 / PB] when tsave is given).  Leaves the panel's unit-lower reflectors in
 // LDS P (rows x PB, rows = m - j0) and T in LDS Tm; returns jb.
 template <typename T, int PB>
-__device__ int wg_geqrf_panel(int m, int ncols, T *A, int64_t lda, T *tau, T *tsave, T *lds, int32_t *piv,
-                              int64_t *hdr, int j0, const T *cn = nullptr) {
+__device__ int wg_geqrf_panel(int m, int ncols, T *A, int64_t lda, T *tau, T *tsave, T *lds, int64_t *hdr,
+                              int j0) {
     (void) hdr;
     T *P = lds;
     T *Tm = P + (int64_t) (m | 1) * PB;
@@ -787,9 +784,6 @@ __device__ int wg_geqrf_panel(int m, int ncols, T *A, int64_t lda, T *tau, T *ts
     const int rows = m - j0;
     const int pld = panel_ld(rows);
     HCAMD_SUB_BEGIN(t_pan);
-    HCAMD_SUB_BEGIN(t_piv);
-    if (piv) window_pivot<T, PB>(m, ncols, A, lda, j0, jb, piv, P, cn);
-    HCAMD_SUB_END(t_piv, hdr, 5);
     // one row per thread and iteration, the PB loads of a row in flight together
     for (int r = threadIdx.x; r < rows; r += NT) {
         T v[PB];
@@ -924,19 +918,15 @@ __device__ int wg_geqrf_panel(int m, int ncols, T *A, int64_t lda, T *tau, T *ts
 // the stacked left factor `src`; the first trailing update reads the others in place and writes
 // them into A.
 template <typename T, int PB>
-__device__ void wg_geqrf(int m, int ncols, T *A, int64_t lda, T *tau, T *tsave, T *lds, int32_t *piv = nullptr,
-                         int64_t *hdr = nullptr, bool from_src = false, StackedU<T> src = StackedU<T>{}) {
+__device__ void wg_geqrf(int m, int ncols, T *A, int64_t lda, T *tau, T *tsave, T *lds, int64_t *hdr = nullptr,
+                         bool from_src = false, StackedU<T> src = StackedU<T>{}) {
     T *P = lds;
     T *Tm = P + (int64_t) (m | 1) * PB;
     T *red = Tm + 2 * PB * PB;
     const int nsteps = m < ncols ? m : ncols;
-    if (piv) {
-        for (int c = threadIdx.x; c < ncols; c += NT) piv[c] = c;
-        __syncthreads();
-    }
     for (int j0 = 0; j0 < nsteps; j0 += PB) {
         const bool first_src = from_src && j0 == 0;
-        const int jb = wg_geqrf_panel<T, PB>(m, ncols, A, lda, tau, tsave, lds, piv, hdr, j0);
+        const int jb = wg_geqrf_panel<T, PB>(m, ncols, A, lda, tau, tsave, lds, hdr, j0);
         HCAMD_SUB_BEGIN(t_up);
         if (j0 + jb < ncols) {
             if constexpr (PB == 16 && sizeof(T) == 8) {
@@ -1013,7 +1003,7 @@ __device__ void ph_qr_y(const RecompDesc<T> &d, T *lds) {
     if (!pivot) {
         for (int c = threadIdx.x; c < z.mu; c += NT) w.piv[c] = c;
         __syncthreads();
-        wg_geqrf<T, PB>(d.n, z.mu, w.y, d.n, w.tau_y, w.t_y, lds, nullptr, w.hdr);
+        wg_geqrf<T, PB>(d.n, z.mu, w.y, d.n, w.tau_y, w.t_y, lds, w.hdr);
         return;
     }
     const int m = d.n, ncols = z.mu;
@@ -1041,7 +1031,7 @@ __device__ void ph_qr_y(const RecompDesc<T> &d, T *lds) {
             __syncthreads();
             return;
         }
-        wg_geqrf_panel<T, PB>(m, ncols, w.y, m, w.tau_y, w.t_y, lds, nullptr, w.hdr, j0);
+        wg_geqrf_panel<T, PB>(m, ncols, w.y, m, w.tau_y, w.t_y, lds, w.hdr, j0);
         if (j0 + jb < ncols)
             apply_wy_dispatch<T, PB>(P, panel_ld(m - j0), Tm, m - j0, w.y + j0, m, j0 + jb, ncols, true, red,
                                      fused_norms ? cn : nullptr, jb);
