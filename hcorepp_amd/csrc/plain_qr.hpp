@@ -102,16 +102,25 @@ __device__ __forceinline__ void store4(float *q, bool wide, const float (&v)[4])
     else q[0] = v[0], q[1] = v[1], q[2] = v[2], q[3] = v[3];
 }
 // Rows r .. r + 3 of a column of `rows` rows, zero (not written) past its end.  Blocks of more than eight groups make every
-// load, at the column's last row where its own is past the end: with branches around them the branches' state took the
-// registers.  (The kernels of 1025 to 2048 rows had 310 to 750 bytes of scratch per lane; below about 270 each launch is 60 us
-// shorter, an update of rank 1 in a 2048 x 2048 tile 260 -> 170 us, of rank 128 6.66 -> 3.28 ms.)
+// load, at the column's last row where its own is past the end (load_any), and clear what was not asked for afterwards: with
+// branches around them the branches' state took the registers.  (The kernels of 1025 to 2048 rows had 310 to 750 bytes of scratch
+// per lane; below about 270 each launch is 60 us shorter, an update of rank 1 in a 2048 x 2048 tile 260 -> 170 us, of rank 128
+// 6.66 -> 3.28 ms.)
+template <typename T>
+__device__ __forceinline__ void load_any(const T *col, int r, int rows, T (&v)[4]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) v[s] = col[r + s < rows ? r + s : rows - 1];
+}
+template <typename T>
+__device__ __forceinline__ void clear_rows(int r, int rows, bool ok, T (&v)[4]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) v[s] = (ok && r + s < rows) ? v[s] : T(0);
+}
 template <int GROUPS, typename T>
 __device__ __forceinline__ void load_rows(const T *col, int r, int rows, bool ok, bool wide, T (&v)[4]) {
     if constexpr (GROUPS > 8) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) v[s] = col[r + s < rows ? r + s : rows - 1];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) v[s] = (ok && r + s < rows) ? v[s] : T(0);
+        load_any(col, r, rows, v);
+        clear_rows(r, rows, ok, v);
     } else if (ok && r + 3 < rows) {
         load4(col + r, wide, v);
     } else {
@@ -149,6 +158,27 @@ template <int GROUPS>
 __device__ __forceinline__ int own_rows(int r) {
     if constexpr (GROUPS > 8) asm volatile("" : "+v"(r));
     return r;
+}
+
+// A wave's rows of a column (groups wave, wave + WAVES, ..).  Past eight groups all loads are made before the first value is
+// looked at: cleared group by group, each group waited for its own (a panel of one column of 2048 rows 26.6 us, 22.0 now).
+template <int WAVES, int GROUPS, typename T>
+__device__ __forceinline__ void load_block(const T *col, int rows, bool ok, bool wide, T (&b)[GROUPS][4]) {
+    const int r0 = 16 * wave_id() + 4 * (lane_id() >> 4);
+#pragma unroll
+    for (int t = 0; t < GROUPS; ++t) {
+        const int r = own_rows<GROUPS>(r0 + 16 * WAVES * t);
+        if constexpr (GROUPS > 8) load_any(col, r, rows, b[t]);
+        else load_rows<GROUPS>(col, r, rows, ok, wide, b[t]);
+        group_end<GROUPS>();
+    }
+    if constexpr (GROUPS > 8) {
+#pragma unroll
+        for (int t = 0; t < GROUPS; ++t) {
+            clear_rows(own_rows<GROUPS>(r0 + 16 * WAVES * t), rows, ok, b[t]);
+            group_end<GROUPS>();
+        }
+    }
 }
 
 __device__ __forceinline__ double rcp_full(double d) {
@@ -449,12 +479,7 @@ __device__ __forceinline__ void wg_panel(const PlainQr<T> &q, int j0, PanelLds<T
     const bool wide = wide_columns(q.A, q.m);
     auto column = [&](int c) { return q.A + (int64_t) (q.pivot ? l.piv[c] : j0 + c) * q.m + j0; };
     T p[GROUPS][4];
-    const T *src = column(i16 < jb ? i16 : 0);
-#pragma unroll
-    for (int t = 0; t < GROUPS; ++t) {
-        load_rows<GROUPS>(src, own_rows<GROUPS>(16 * (wv + WAVES * t) + 4 * k4), rows, i16 < jb, wide, p[t]);
-        group_end<GROUPS>();
-    }
+    load_block<WAVES>(column(i16 < jb ? i16 : 0), rows, i16 < jb, wide, p);
     const T scal = panel_factor<T, WAVES, GROUPS>(p, jb, q.tau + j0, l);
     const int c = (i16 + jb) & 15;
     T *dst = column(c < jb ? c : 0);
