@@ -242,7 +242,7 @@ struct PanelLds {
 //
 // Bound by the chain of a column: two reductions' latency, a reciprocal square root and a reciprocal, one
 // barrier: 0.7 us per column up to 512 rows.  Lanes along the columns need two exchanges per sum where a row
-// per lane took six for 16 values.  A whole panel of the pivoted QR takes 20 us at 256 rows and 36 at 1024
+// per lane took six for 16 values.  A whole panel of the pivoted QR takes 20 us at 256 rows and 37 at 1024
 // (50 and 47, for half as many columns, in LDS with a row per thread and four waves), its trailing update 7 and 18.
 template <typename T, int WAVES, int GROUPS>
 __device__ __forceinline__ T panel_factor(T (&p)[GROUPS][4], int jb, T *tau, PanelLds<T, WAVES> &l) {
